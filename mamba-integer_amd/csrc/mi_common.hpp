@@ -153,6 +153,19 @@ __device__ __forceinline__ void update16_cs_first(int32_t &h, int n2, int b, int
     asm("" : "+v"(yhi), "+v"(ylo));
 }
 
+// sat32(b * x + d) for the int16 halves `half` (0 low, 1 high) of bw and xw:
+// v_mad_i32_i16 with the clamp bit saturates the full-precision sum (checked on
+// the hardware against a 64-bit saturating reference, every operand half)
+template <int kHalf>
+__device__ __forceinline__ int mad16_sat(int bw, int xw, int d) {
+    int r;
+    if constexpr (kHalf == 0)
+        asm("v_mad_i32_i16 %0, %1, %2, %3 clamp" : "=v"(r) : "v"(bw), "v"(xw), "v"(d));
+    else
+        asm("v_mad_i32_i16 %0, %1, %2, %3 op_sel:[1,1,0,0] clamp" : "=v"(r) : "v"(bw), "v"(xw), "v"(d));
+    return r;
+}
+
 // Exact floor(sqrt(v)) for v < 2^62 (host and device): a float estimate
 // refined by integer correction steps.
 __host__ __device__ __forceinline__ uint64_t isqrt64(uint64_t v) {
@@ -221,6 +234,27 @@ constexpr int32_t dt_q16_table_entry(int dm) {
     const int64_t s = (int64_t)dm * 65536 + (int64_t)isqrt64_bitwise((uint64_t)((int64_t)dm * dm) * (1ull << 32) +
                                                                      (1ull << 34));
     return (int32_t)clamp64(rshr64(655 * (s >> 1), 16), 66, 6554);
+}
+
+// Q7 unit-vector scale of spec rule 7.4 from the row's sum of squares: floor(2^30 /
+// isqrt(ss * 2^16)), for ss < 2^22 (256 states of int8).  ss * 2^16 is exact in
+// float and its root is below 2^19, so v_sqrt_f32's last-place error leaves the
+// truncated root within one; the reciprocal's (2^-23 of a quotient of at most
+// 2^22) leaves the quotient within one.  One compare each way makes both exact.
+__device__ __forceinline__ int32_t unit_inv(int32_t ss) {
+    if (ss == 0) return 0;
+    const uint64_t v = (uint64_t)(uint32_t)ss << 16;
+    uint32_t s = (uint32_t)__builtin_amdgcn_sqrtf((float)ss * 65536.0f);
+    s -= (uint64_t)s * s > v ? 1u : 0u;
+    s += (uint64_t)(s + 1) * (s + 1) <= v ? 1u : 0u;
+    uint32_t q = (uint32_t)(1073741824.0f * __builtin_amdgcn_rcpf((float)s));
+    int32_t r = (int32_t)((1u << 30) - q * s);
+    if (r < 0) {
+        --q;
+        r += (int32_t)s;
+    }
+    if (r >= (int32_t)s) ++q;
+    return (int32_t)q;
 }
 
 // Gate of spec rule 4.11 (mamba_integer_model.py:124-132), Q15, z in Q4.
