@@ -147,72 +147,168 @@ __global__ __launch_bounds__(256) void scan_f32_kernel(const float *x, const int
     }
 }
 
-// Elementwise integer recurrence: one lane per (b, channel), int32 state.
-__global__ __launch_bounds__(256) void scan_elem_kernel(const int32_t *u, const int32_t *n, int k, int32_t *h,
-                                                        const int32_t *h_in, int32_t *h_out, int B, int L, int C) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)B * C) return;
-    const int c = (int)(idx % C);
-    const int b = (int)(idx / C);
-    int32_t s = h_in ? h_in[idx] : 0;
-    for (int t = 0; t < L; ++t) {
-        const int64_t off = ((int64_t)b * L + t) * C + c;
-        s = sat32_64((((int64_t)s * n[off]) >> k) + (int64_t)u[off]);
-        h[off] = s;
+// Elementwise integer recurrence over u, n [B][L][C] (DyadicScanFunction, and with
+// CHUNKED the per-chunk outputs of ssd_chunked_scan_forward, ssd_chunked_scan.py:
+// 382-422: the state at each chunk's last step and the chunk's cumulative decay
+// in Q30, 2^30 decayed by the chunk's steps and rounded down after each).
+//
+// Bound: HBM (12 bytes a step and channel) where enough bytes are in flight,
+// else the chain of steps.  With one lane per channel a load brings 4 bytes a
+// lane of one step, and a wave can have 63 memory operations outstanding: about
+// 20 steps, so a memory latency every 20 steps bounds small channel counts.  Here
+// a wave owns 64 / R channels and its R rows of lanes load R consecutive steps at
+// once (kElemAhead groups of R steps in registers).  Every row then runs all R
+// steps: the rows' operands are exchanged by v_permlane16/32_swap, and row r
+// keeps step r's state for one store per group.  The update is the 64-bit
+// product, its shift and a clamped add when every decay of the group lies in
+// [0, 2^k] (a vote), else the saturating 64-bit form.  B1 x L2048 x 24576 channels
+// 963 -> 146 us (4.1 TB/s); chunked B4 x L1000 x 1536 145 -> 56 us.
+constexpr int kElemAhead = 16;
+
+// Every row's value of v for all rows: o[i] = v of row i (R rows of 64 / R lanes).
+template <int R>
+__device__ __forceinline__ void row_values(int v, int (&o)[R]) {
+    if constexpr (R == 1) {
+        o[0] = v;
+    } else if constexpr (R == 2) {
+        const auto ab = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+        o[0] = (int)ab[0];
+        o[1] = (int)ab[1];
+    } else {
+        const auto ab = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);   // (a a c c), (b b d d)
+        const auto ac = __builtin_amdgcn_permlane32_swap(ab[0], ab[0], false, false);
+        const auto bd = __builtin_amdgcn_permlane32_swap(ab[1], ab[1], false, false);
+        o[0] = (int)ac[0];
+        o[1] = (int)bd[0];
+        o[2] = (int)ac[1];
+        o[3] = (int)bd[1];
     }
-    if (h_out) h_out[idx] = s;
 }
 
-// Chunked elementwise recurrence with the per-chunk outputs of
-// ssd_chunked_scan_forward (ssd_chunked_scan.py:382-422): one lane per
-// (b, channel), its steps in order.  The operands of kAhead steps are loaded
-// before the dependent chain runs over them, from clamped in-bounds addresses
-// (no per-lane condition, so the loads issue back to back); a step past the
-// end is skipped by a branch that is uniform across the block.  At the end of
-// each chunk the lane stores its state and the chunk's cumulative decay in
-// Q30 (2^30 decayed by the chunk's steps, rounded down after each step).
-constexpr int kAhead = 8;
-__global__ __launch_bounds__(64) void chunked_scan_kernel(const int32_t *__restrict__ u, const int32_t *__restrict__ n,
-                                                          int k, int cs, int32_t *__restrict__ h,
-                                                          int32_t *__restrict__ final_h, int32_t *__restrict__ dte,
-                                                          const int32_t *h_in, int32_t *h_out, int B, int L, int C,
-                                                          int nc) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)B * C) return;
-    const int c = (int)(idx % C);
-    const int b = (int)(idx / C);
-    const int64_t base = (int64_t)b * L * C + c;
-    int32_t s = h_in ? h_in[idx] : 0;
+template <bool CHUNKED, int R, int W>
+__global__ __launch_bounds__(64 * W) void elem_scan_kernel(const int32_t *u, const int32_t *n, int k, int cs, int32_t *h,
+                                                           int32_t *final_h, int32_t *dte, const int32_t *h_in,
+                                                           int32_t *h_out, int L, int C, int cblocks, int nc) {
+    constexpr int CW = 64 / R;                    // channels of a wave
+    const int lane = threadIdx.x & 63, r = lane / CW;
+    const int64_t b = blockIdx.x / cblocks;
+    const int c0 = ((int)(blockIdx.x % cblocks) * W + wave_id()) * CW;
+    if (c0 >= C) return;
+    const int c = min(c0 + lane % CW, C - 1);     // lanes past the end repeat the last channel, values and stores alike
+    int32_t s = h_in ? h_in[b * C + c] : 0;
     int32_t p = 1 << 30;
-    int left = cs;     // steps left in the current chunk
-    int chunk = 0;
-    for (int t0 = 0; t0 < L; t0 += kAhead) {
-        int32_t uu[kAhead], nn[kAhead];
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j) {
-            const int64_t off = base + (int64_t)min(t0 + j, L - 1) * C;
-            uu[j] = u[off];
-            nn[j] = n[off];
+    int left = cs, chunk = 0;                     // steps left in the chunk
+    const uint32_t lim = 1u << k;
+
+    const int64_t base = b * L * C;
+    const uint32_t off = (uint32_t)r * (uint32_t)C + (uint32_t)c;
+    const int groups = L / R;                     // whole ones
+    auto row = [&](const int32_t *q, int g) { return q + base + (int64_t)g * R * C + off; };
+    auto step = [&](int uv, int nv, bool fast) {
+        if (fast) {
+            s = __builtin_elementwise_add_sat((int32_t)(((int64_t)s * nv) >> k), uv);
+            if constexpr (CHUNKED) p = (int32_t)(((int64_t)p * nv) >> k);
+        } else {
+            s = sat32_64((((int64_t)s * nv) >> k) + (int64_t)uv);
+            if constexpr (CHUNKED) p = sat32_64(((int64_t)p * nv) >> k);
         }
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j) {
-            const int t = t0 + j;
-            if (t < L) {
-                s = sat32_64((((int64_t)s * nn[j]) >> k) + (int64_t)uu[j]);
-                h[base + (int64_t)t * C] = s;
-                p = sat32_64(((int64_t)p * nn[j]) >> k);
-                if (--left == 0 || t + 1 == L) {
-                    const int64_t co = ((int64_t)b * nc + chunk) * C + c;
-                    if (final_h) final_h[co] = s;
-                    if (dte) dte[co] = p;
-                    p = 1 << 30;
-                    left = cs;
-                    ++chunk;
-                }
+    };
+    // after `steps` steps, the last of them the chunk's or the sequence's: wave-uniform
+    auto chunk_end = [&](int steps, bool last) {
+        left -= steps;
+        if (left == 0 || last) {
+            const int64_t co = (b * nc + chunk) * C + c;
+            if (r == 0) {
+                if (final_h) final_h[co] = s;
+                if (dte) dte[co] = p;
             }
+            p = 1 << 30;
+            left = cs;
+            ++chunk;
+        }
+    };
+    int32_t uu[kElemAhead], nn[kElemAhead];
+    if (groups > 0) {
+#pragma unroll
+        for (int j = 0; j < kElemAhead; ++j) {
+            uu[j] = *row(u, min(j, groups - 1));
+            nn[j] = *row(n, min(j, groups - 1));
         }
     }
-    if (h_out) h_out[idx] = s;
+    auto group = [&](int32_t uv, int32_t nv, int g) {
+        int ur[R], nr[R];
+        row_values<R>(uv, ur);
+        row_values<R>(nv, nr);
+        int keep = 0;
+        if (!__any((uint32_t)nv > lim)) {
+#pragma unroll
+            for (int e = 0; e < R; ++e) {
+                step(ur[e], nr[e], true);
+                keep = r == e ? s : keep;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < R; ++e) {
+                step(ur[e], nr[e], false);
+                keep = r == e ? s : keep;
+            }
+        }
+        *const_cast<int32_t *>(row(h, g)) = keep;
+        if constexpr (CHUNKED) chunk_end(R, g * R + R == L);   // (R divides the chunk length)
+    };
+    // whole rounds of kElemAhead groups (no exits inside: the register arrays
+    // would be copied at each), then the last groups, already loaded
+    int g0 = 0;
+    for (; g0 + kElemAhead <= groups; g0 += kElemAhead) {
+#pragma unroll
+        for (int j = 0; j < kElemAhead; ++j) {
+            const int32_t uv = uu[j], nv = nn[j];
+            const int nx = min(g0 + j + kElemAhead, groups - 1);   // past the end: the last group again, unused
+            uu[j] = *row(u, nx);
+            nn[j] = *row(n, nx);
+            group(uv, nv, g0 + j);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kElemAhead - 1; ++j)
+        if (g0 + j < groups) group(uu[j], nn[j], g0 + j);
+    for (int t = R * groups; t < L; ++t) {   // fewer than R steps, every row the same
+        const int64_t o = base + (int64_t)t * C + c;
+        const int nv = n[o];
+        step(u[o], nv, false);
+        if (r == 0) h[o] = s;
+        if constexpr (CHUNKED) chunk_end(1, t + 1 == L);
+    }
+    if (h_out && r == 0) h_out[b * C + c] = s;
+}
+
+template <bool CHUNKED, int R, int W>
+void launch_elem_rows(const int32_t *u, const int32_t *n, int k, int cs, int32_t *h, int32_t *final_h, int32_t *dte,
+                      const int32_t *h_in, int32_t *h_out, int B, int L, int C, int nc, hipStream_t st) {
+    constexpr int CB = 64 / R * W;   // channels of a block
+    const int64_t cb = ((int64_t)C + CB - 1) / CB;
+    hipLaunchKernelGGL((elem_scan_kernel<CHUNKED, R, W>), dim3((unsigned)(cb * B)), dim3(64 * W), 0, st, u, n, k, cs, h,
+                       final_h, dte, h_in, h_out, L, C, (int)cb, nc);
+}
+template <bool CHUNKED>
+void launch_elem_scan(const int32_t *u, const int32_t *n, int k, int cs, int32_t *h, int32_t *final_h, int32_t *dte,
+                      const int32_t *h_in, int32_t *h_out, int B, int L, int C, int nc, hipStream_t st) {
+    // Rows of steps by the channels there are: four where the waves are few (each
+    // then has the most steps in flight), two and one, whose accesses are whole
+    // 128- and 256-byte lines, where there are enough waves without.  us for
+    // four / two / one (elementwise): 6144 channels x 1000 steps 45 / 62 / 81, 16384
+    // x 2048 104 / 142 / 192, 24576 x 2048 183 / 146 / 200, 65536 x 2048 432 / 319 /
+    // 293.  A chunk ends with a group: fewer rows where four do not divide it.
+    const int64_t lanes = (int64_t)B * C;
+    const int rows = lanes >= 49152 ? 1 : lanes >= 20480 ? 2 : 4;
+    const int even = !CHUNKED || cs % 4 == 0 ? 4 : cs % 2 == 0 ? 2 : 1;
+    auto go = [&](auto f) { f(u, n, k, cs, h, final_h, dte, h_in, h_out, B, L, C, nc, st); };
+    if (rows == 4 && even == 4)
+        go(lanes > 8192 ? launch_elem_rows<CHUNKED, 4, 4> : launch_elem_rows<CHUNKED, 4, 2>);
+    else if (rows >= 2 && even >= 2)
+        go(launch_elem_rows<CHUNKED, 2, 4>);
+    else
+        go(launch_elem_rows<CHUNKED, 1, 4>);
 }
 
 }  // namespace
@@ -365,9 +461,8 @@ extern "C" mi_status mi_dyadic_scan_elementwise(const int32_t *u, const int32_t 
     if ((int64_t)batch * channels == 0 || (len == 0 && !h_out)) return MI_OK;
     MI_REQUIRE(len == 0 || (u && nums && h), MI_ERR_NULL_POINTER,
                "mi_dyadic_scan_elementwise: u, nums and h are required");
-    const int64_t lanes = (int64_t)batch * channels;
-    hipLaunchKernelGGL(scan_elem_kernel, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, as_stream(stream), u,
-                       nums, decay_shift, h, h_in, h_out, batch, len, channels);
+    launch_elem_scan<false>(u, nums, decay_shift, 0, h, nullptr, nullptr, h_in, h_out, batch, len, channels, 0,
+                            as_stream(stream));
     return check_launch("mi_dyadic_scan_elementwise");
 }
 
@@ -382,9 +477,8 @@ extern "C" mi_status mi_dyadic_chunked_scan(const int32_t *u, const int32_t *num
     // len == 0 with h_out: the kernel runs no step and writes h_out = h_in (zeros when NULL)
     if ((int64_t)batch * channels == 0 || (len == 0 && !h_out)) return MI_OK;
     MI_REQUIRE(len == 0 || (u && nums && h), MI_ERR_NULL_POINTER, "mi_dyadic_chunked_scan: u, nums and h are required");
-    const int64_t lanes = (int64_t)batch * channels;
     const int nc = (int)((len + (int64_t)chunk - 1) / chunk);
-    hipLaunchKernelGGL(chunked_scan_kernel, dim3((unsigned)((lanes + 63) / 64)), dim3(64), 0, as_stream(stream), u,
-                       nums, decay_shift, chunk, h, final_h, decay_to_end, h_in, h_out, batch, len, channels, nc);
+    launch_elem_scan<true>(u, nums, decay_shift, chunk, h, final_h, decay_to_end, h_in, h_out, batch, len, channels, nc,
+                           as_stream(stream));
     return check_launch("mi_dyadic_chunked_scan");
 }

@@ -30,6 +30,8 @@ import torch
 
 from mamba_int import ops
 
+_Q30 = torch.tensor(2.0 ** -30, dtype=torch.float32)
+
 
 def _shift(shifts: Union[int, torch.Tensor]) -> int:
     if not isinstance(shifts, torch.Tensor):
@@ -56,7 +58,7 @@ def ssd_chunked_scan_forward(u: torch.Tensor, nums: torch.Tensor, shifts, chunk_
         raise TypeError("the integer chunked scan takes integer decay numerators")
     h, final_h, dte_q30 = ops.dyadic_chunked_scan(u.contiguous(), nums.to(torch.int32).contiguous(),
                                                   _shift(shifts), int(chunk_size))
-    return h, final_h, dte_q30.to(torch.float32) * (1.0 / (1 << 30))
+    return h, final_h, dte_q30 * _Q30      # int32 -> float32 and the exact scale in one kernel
 
 
 class SSDChunkedScanFunction:
