@@ -142,6 +142,15 @@ mi_status mi_pack_ternary(const int8_t *w, uint8_t *packed, int n, int k, void *
 mi_status mi_act_quant_f32(const float *x, int8_t *xq, float *x_scale, int m, int k,
                            void *stream);
 
+/* BitLinear.forward on fp32 rows (rational_bitnet.py:167-213): mi_act_quant_f32
+ * of x [m,k] into xq int8 [m,kp] (columns from k on zero) and x_scale [m], then
+ * mi_bitlinear MI_OUT_FLOAT over w_packed [n, kp/4] (k padded to kp with zero
+ * weights; kp % 16 == 0), plus bias fp32 [n] (nullable) added after the scale.
+ * xq (16-byte aligned) and x_scale are scratch that the caller owns. */
+mi_status mi_bitlinear_f32(const float *x, int k, const uint8_t *w_packed, int kp, float w_scale,
+                           const float *bias, int8_t *xq, float *x_scale, float *out, int ldo,
+                           int m, int n, void *stream);
+
 /* out[m, n] = kind(sum_k a[m,k] * W[n,k]) (replaces BitLinear.forward's
  * F.linear + rescale, rational_bitnet.py:204-208, and launch_bitlinear).
  * a int8 [m, lda] (16-byte aligned, lda % 16 == 0); w_packed [n, k/4]

@@ -31,6 +31,7 @@ SIGNATURES = {
     "mi_ssd_chunked_scan": [P, P, P, P, I, P, P, P, P, I, I, I, I, I, I, P],
     "mi_pack_ternary": [P, P, I, I, P],
     "mi_act_quant_f32": [P, P, P, I, I, P],
+    "mi_bitlinear_f32": [P, I, P, I, F, P, P, P, P, I, I, I, P],
     "mi_bitlinear": [P, I, P, P, I, I, I, I, I, I, I32, I, I32, P, F, P, P],
     "mi_bitlinear_gemm": [P, I, P, P, I, I, I, I, I, I, I32, I, I32, P, F, P, P],
     "mi_bitlinear_gemv": [P, I, P, P, I, I, I, I, I, I, I32, I, I32, P, F, P, P],

@@ -163,6 +163,23 @@ def bitlinear(a: torch.Tensor, w_packed: torch.Tensor, kind: int, n: int, k: Opt
     return out
 
 
+def bitlinear_f32(x: torch.Tensor, w_packed: torch.Tensor, w_scale: float,
+                  bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """BitLinear.forward on fp32 rows x [m, k]: quantize (padded to the packed weights' k with
+    zeros), product, scale and bias -> fp32 [m, n]."""
+    _req(x, torch.float32, "x"); _req(w_packed, torch.uint8, "w_packed")
+    m, k = x.shape
+    n, kp = w_packed.shape[0], 4 * w_packed.shape[1]
+    if bias is not None and _req(bias, torch.float32, "bias").numel() != n:
+        raise ValueError(f"bias must have {n} elements, got {bias.numel()}")
+    xq = torch.empty((m, kp), dtype=torch.int8, device=x.device)
+    x_scale = torch.empty((m,), dtype=torch.float32, device=x.device)
+    out = torch.empty((m, n), dtype=torch.float32, device=x.device)
+    _lib.call("mi_bitlinear_f32", _ptr(x), k, _ptr(w_packed), kp, ctypes.c_float(w_scale), _ptr(bias), _ptr(xq),
+              _ptr(x_scale), _ptr(out), n, m, n, _stream())
+    return out
+
+
 # ---------------------------------------------------------------- block ops
 def bitshift_norm(r: torch.Tensor, gamma: torch.Tensor, out=None, row_stats=None, v2: bool = False) -> torch.Tensor:
     """Integer BitShiftNorm of r int32 [T, d]; v2 selects BitShiftNormV2's table.  row_stats:

@@ -52,8 +52,8 @@ def activation_quant_dynamic(x: torch.Tensor, bits: int = 8) -> Tuple[torch.Tens
     return q.to(torch.float32).view(shape), s.view(*shape[:-1], 1)
 
 
-def _ceil16(k: int) -> int:
-    return (k + 15) // 16 * 16
+def _ceil(k: int, unit: int) -> int:
+    return (k + unit - 1) // unit * unit
 
 
 class BitLinear(nn.Module):
@@ -74,22 +74,23 @@ class BitLinear(nn.Module):
             self.bias = nn.Parameter(torch.zeros(out_features))
         else:
             self.register_parameter("bias", None)
-        self._packed = None
-        self._w_scale = None
+        self._packed = {}        # k unit -> (packed weights, scale)
         self._packed_key = None
 
     # ------------------------------------------------------------ weights
-    def _packed_weights(self, device) -> Tuple[torch.Tensor, float]:
+    def _packed_weights(self, device, unit: int) -> Tuple[torch.Tensor, float]:
+        """The packed ternary weights with k padded to a multiple of ``unit`` (16: the
+        packing unit, the width of ``forward_int``'s rows; 64: four packed words,
+        which the kernels read at once), and their scale; kept per weight version."""
         key = (self.weight._version, self.weight.data_ptr(), str(device))
-        if self._packed is None or self._packed_key != key:
+        if self._packed_key != key:
+            self._packed, self._packed_key = {}, key
+        if unit not in self._packed:
             w_quant, w_scale = weight_quant_ternary(self.weight.detach().to("cpu", torch.float32))
-            k_pad = _ceil16(self.in_features)
-            wq = torch.zeros((self.out_features, k_pad), dtype=torch.int8)
+            wq = torch.zeros((self.out_features, _ceil(self.in_features, unit)), dtype=torch.int8)
             wq[:, : self.in_features] = w_quant.to(torch.int8)
-            self._packed = ops.pack_ternary(wq.to(device))
-            self._w_scale = float(w_scale)
-            self._packed_key = key
-        return self._packed, self._w_scale
+            self._packed[unit] = ops.pack_ternary(wq.to(device)), float(w_scale)
+        return self._packed[unit]
 
     @torch.no_grad()
     def get_ternary_weights(self) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -97,15 +98,6 @@ class BitLinear(nn.Module):
         return w_quant.to(torch.int8), w_scale
 
     # ------------------------------------------------------------ forward
-    def _quantized_input(self, x2: torch.Tensor):
-        xq, x_scale = ops.act_quant(x2)
-        k_pad = _ceil16(self.in_features)
-        if k_pad != self.in_features:
-            padded = torch.zeros((xq.shape[0], k_pad), dtype=torch.int8, device=xq.device)
-            padded[:, : self.in_features] = xq
-            xq = padded
-        return xq, x_scale
-
     @torch.no_grad()
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not x.is_cuda:
@@ -114,15 +106,18 @@ class BitLinear(nn.Module):
             raise ValueError("the integer path quantizes activations to 8 bits")
         shape = x.shape
         x2 = x.reshape(-1, self.in_features).to(torch.float32).contiguous()
-        packed, w_scale = self._packed_weights(x.device)
-        xq, x_scale = self._quantized_input(x2)
-        y = ops.bitlinear(xq, packed, ops.OUT_FLOAT, self.out_features, x_scale=x_scale, w_scale=w_scale)
-        if self.bias is not None:
-            y = y + self.bias.to(y.device)
+        packed, w_scale = self._packed_weights(x.device, 64)
+        bias = self.bias
+        # a float32 bias of the device is added by the GEMM's epilogue, any other
+        # by torch (with its promotion)
+        fused = bias is not None and bias.dtype == torch.float32 and bias.device == x.device and bias.is_contiguous()
+        y = ops.bitlinear_f32(x2, packed, w_scale, bias=bias if fused else None)
+        if bias is not None and not fused:
+            y = y + bias.to(y.device)
         return y.view(*shape[:-1], self.out_features)
 
     @torch.no_grad()
     def forward_int(self, a: torch.Tensor, kind: int = ops.OUT_INT32, shift: int = 0) -> torch.Tensor:
         """Integer face: a int8 [M, K] (K = in_features padded to 16) -> acc / requantized int8."""
-        packed, _ = self._packed_weights(a.device)
+        packed, _ = self._packed_weights(a.device, 16)
         return ops.bitlinear(a.contiguous(), packed, kind, self.out_features, shift=shift)
