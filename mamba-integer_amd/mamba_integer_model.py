@@ -273,7 +273,7 @@ class MambaIntegerModel(nn.Module):
     def forward(self, input_ids: torch.Tensor) -> torch.Tensor:
         if not input_ids.is_cuda:
             raise ValueError("MambaIntegerModel runs on the GPU; move input_ids to the device")
-        return self.forward_int(input_ids).to(torch.float32) * self.logit_scale
+        return self.runner(input_ids.device).forward_float(input_ids, self.logit_scale)
 
     @torch.no_grad()
     def generate(self, input_ids: torch.Tensor, max_new_tokens: int, use_graph: bool = True) -> torch.Tensor:
