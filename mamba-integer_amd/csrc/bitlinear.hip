@@ -19,10 +19,13 @@
 //                 stay packed in LDS and are unpacked in registers), double
 //                 buffered, one barrier per stage (gemm_kernel); from 512 tiles
 //                 up 256(n) x 128(m) tiles on 32x32x32 MFMAs with an LDS-DMA
-//                 ring (gemm32_kernel).
+//                 ring (gemm32_kernel); for few tokens or features 64 x 64
+//                 tiles on such a ring (gemm_ring_kernel).
 //   decode GEMV:  m <= 64; a block owns 16 output features, its 4 waves split
 //                 K; each lane streams 16-byte words of packed weights straight
 //                 from HBM and unpacks them in registers.
+#include <algorithm>
+
 #include "mi_mfma.hpp"
 
 namespace mi {
@@ -41,6 +44,7 @@ struct GemmArgs {
     int32_t res_mult;
     int res_shift;
     int32_t res_clamp;   // RESIDUAL: |acc| bound before the residual factor (INT32_MAX: none)
+    bool res32;          // RESIDUAL: the increment fits 32 bits for every accumulator (make_args)
     float w_scale;
     int64_t *row_stats;  // RESIDUAL: per-row (sum r, sum r^2) of the new residual, atomically added
     int64_t *stats_parts;  // RESIDUAL: [M][N/16][2] per-block (sum r, sum r^2), plain stores
@@ -60,6 +64,30 @@ typedef __attribute__((address_space(1))) void global_void_t;
 __device__ __forceinline__ int64_t residual_delta(const GemmArgs &g, int32_t acc) {
     const int32_t c = clamp32(acc, -g.res_clamp, g.res_clamp);
     return rshr64((int64_t)c * g.res_mult, g.res_shift);
+}
+
+// The new residual values of 4 consecutive features.  res32 (set by the host
+// where every increment fits 32 bits): one 32 x 32 + 64 multiply-add with the
+// rounding constant, one v_alignbit for the shift, and a saturating 32-bit add
+// in place of the 64-bit shift, add and clamp (6 instructions a value, not
+// ~20; gemm_kernel, 16384 x 1536 -> 768: 38.7 -> 36.9 us).
+__device__ __forceinline__ v4i residual4(const GemmArgs &g, v4i old, v4i acc) {
+    v4i nv;
+    if (g.res32) {
+        const int64_t half = (int64_t)1 << (g.res_shift - 1);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t v = (int64_t)clamp32(acc[r], -g.res_clamp, g.res_clamp) * g.res_mult + half;
+            const int32_t d = (int32_t)__builtin_amdgcn_alignbit((uint32_t)((uint64_t)v >> 32), (uint32_t)v,
+                                                                 (uint32_t)g.res_shift);
+            nv[r] = clamp32(__builtin_elementwise_add_sat(old[r], d), -kResidualLimit, kResidualLimit);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            nv[r] = (int32_t)clamp64((int64_t)old[r] + residual_delta(g, acc[r]), -kResidualLimit, kResidualLimit);
+    }
+    return nv;
 }
 
 // FLOAT outputs of features n .. n + 3: fp32(acc) * (w_scale * x_scale[m]) (rational_bitnet.py:208),
@@ -186,6 +214,58 @@ struct ConvArgs {
     int D, L;               // d_inner, tokens per sequence (M = batch * L)
     int x_blocks;           // ceil(M / kConvRows) * D / kBN
 };
+
+// Depthwise conv + squareplus (spec rules 4.3-4.4) down staged rows [i0, i1)
+// of a tile whose row 0 is token row m0 (i0 >= 3, m0 >= -3), for channels
+// ch..ch+3 with taps tw and biases tb: walks token positions t of sequence sb;
+// the window rows before a sequence start come from the conv state.  row(i):
+// the four in_proj outputs of staged row i.
+template <class Row>
+__device__ __forceinline__ void conv_rows(const ConvArgs &cv, int M, int m0, int i0, int i1, int ch,
+                                          const uint32_t (&tw)[4], const int32_t (&tb)[4], Row row) {
+    int gm = m0 + i0;
+    if (gm >= M) return;
+    int sb = gm / cv.L, t = gm - sb * cv.L;
+    auto state = [&](int k) -> uint32_t {  // x[k] of sequence sb, k in [-3, -1]
+        return cv.st_in ? *reinterpret_cast<const uint32_t *>(cv.st_in + ((int64_t)sb * 3 + 3 + k) * cv.D + ch) : 0u;
+    };
+    // per-channel windows: byte j of win[r] is x[t - 3 + j] of channel ch + r
+    // once row t is shifted in (v_perm_b32 drops byte 0 and appends the new
+    // row's byte r), so the conv is one v_dot4
+    uint32_t win[4] = {0, 0, 0, 0};
+    auto push = [&](uint32_t v) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            win[r] = __builtin_amdgcn_perm(v, win[r], 0x00030201u | ((uint32_t)(4 + r) << 24));
+    };
+    // the window of the run's first row: rows of its own sequence, the conv
+    // state before the sequence start
+    for (int j = 3; j >= 1; --j) push(t - j >= 0 ? row(i0 - j) : state(t - j));
+    for (int i = i0; i < i1 && gm < M; ++i, ++gm) {
+        if (t == 0) {
+            if (i > i0)
+                for (int j = 3; j >= 1; --j) push(state(-j));
+            // a sequence shorter than the window keeps part of the old state
+            for (int j = 0; j < 3 - cv.L; ++j)
+                *reinterpret_cast<uint32_t *>(cv.st_out + ((int64_t)sb * 3 + j) * cv.D + ch) = state(cv.L + j - 3);
+        }
+        const uint32_t cur = row(i);
+        push(cur);
+        uint32_t o = 0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int32_t c = __builtin_amdgcn_sdot4((int)win[r], (int)tw[r], tb[r], false);
+            o |= (uint32_t)(sqp_q(c) & 255) << (8 * r);
+        }
+        *reinterpret_cast<uint32_t *>(cv.xs + (int64_t)gm * cv.D + ch) = o;
+        if (t >= cv.L - 3)
+            *reinterpret_cast<uint32_t *>(cv.st_out + ((int64_t)sb * 3 + t - (cv.L - 3)) * cv.D + ch) = cur;
+        if (++t == cv.L) {
+            t = 0;
+            ++sb;
+        }
+    }
+}
 
 // Tile t of an mtiles x ntiles grid in groups of kGroupM m-tiles: within a
 // group the m-tile runs fastest and the n-tiles sweep (a bijection on
@@ -379,59 +459,11 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const ConvArgs &cv)
         __syncthreads();
         if constexpr (CONV) {
             if (xblk) {
-                // depthwise conv + squareplus (spec rules 4.3-4.4) down the tile:
                 // thread (cg, run) takes channels ch..ch+3 of staged rows
-                // 3 + 16 run .. (16 rows; the last run 13), walking token
-                // positions t of sequence sb; the window rows before a
-                // sequence start come from the conv state
+                // 3 + 16 run .. (16 rows; the last run 13)
                 const int run = tid >> 5;
-                const int i0 = 3 + 16 * run, i1 = min(i0 + 16, kBM);
-                int gm = m0 + i0;   // >= 0: m0 >= -3
-                if (gm < g.M) {
-                    int sb = gm / cv.L, t = gm - sb * cv.L;
-                    auto row = [&](int i) { return *reinterpret_cast<const uint32_t *>(&sO[i * kOpitch + 4 * cg]); };
-                    auto state = [&](int k) -> uint32_t {  // x[k] of sequence sb, k in [-3, -1]
-                        return cv.st_in ? *reinterpret_cast<const uint32_t *>(cv.st_in + ((int64_t)sb * 3 + 3 + k) * cv.D + ch)
-                                        : 0u;
-                    };
-                    // per-channel windows: byte j of win[r] is x[t - 3 + j] of channel
-                    // ch + r once row t is shifted in (v_perm_b32 drops byte 0 and
-                    // appends the new row's byte r), so the conv is one v_dot4
-                    uint32_t win[4] = {0, 0, 0, 0};
-                    auto push = [&](uint32_t v) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            win[r] = __builtin_amdgcn_perm(v, win[r], 0x00030201u | ((uint32_t)(4 + r) << 24));
-                    };
-                    // the window of the run's first row: rows of its own sequence, the
-                    // conv state before the sequence start
-                    for (int j = 3; j >= 1; --j) push(t - j >= 0 ? row(i0 - j) : state(t - j));
-                    for (int i = i0; i < i1 && gm < g.M; ++i, ++gm) {
-                        if (t == 0) {
-                            if (i > i0)
-                                for (int j = 3; j >= 1; --j) push(state(-j));
-                            // a sequence shorter than the window keeps part of the old state
-                            for (int j = 0; j < 3 - cv.L; ++j)
-                                *reinterpret_cast<uint32_t *>(cv.st_out + ((int64_t)sb * 3 + j) * cv.D + ch) =
-                                    state(cv.L + j - 3);
-                        }
-                        const uint32_t cur = row(i);
-                        push(cur);
-                        uint32_t o = 0;
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int32_t c = __builtin_amdgcn_sdot4((int)win[r], (int)tw[r], tb[r], false);
-                            o |= (uint32_t)(sqp_q(c) & 255) << (8 * r);
-                        }
-                        *reinterpret_cast<uint32_t *>(cv.xs + (int64_t)gm * cv.D + ch) = o;
-                        if (t >= cv.L - 3)
-                            *reinterpret_cast<uint32_t *>(cv.st_out + ((int64_t)sb * 3 + t - (cv.L - 3)) * cv.D + ch) = cur;
-                        if (++t == cv.L) {
-                            t = 0;
-                            ++sb;
-                        }
-                    }
-                }
+                conv_rows(cv, g.M, m0, 3 + 16 * run, min(19 + 16 * run, kBM), ch, tw, tb,
+                          [&](int i) { return *reinterpret_cast<const uint32_t *>(&sO[i * kOpitch + 4 * cg]); });
                 return;
             }
         }
@@ -479,23 +511,20 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const ConvArgs &cv)
                 for (int i = 0; i < NI; ++i) {
                     const int n = n0 + nb + i * 16 + 4 * lq;
                     if (m < g.M && n < g.N) {
-                        v4i nv;
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int64_t delta = residual_delta(g, acc[i][j][r]);
-                            nv[r] = (int32_t)clamp64((int64_t)old[jj][i][r] + delta, -kResidualLimit, kResidualLimit);
-                        }
+                        const v4i nv = residual4(g, old[jj][i], acc[i][j]);
                         int32_t *o = ob + (int64_t)m * g.ldo + n;
                         if (n + 3 < g.N) {
                             *reinterpret_cast<v4i *>(o) = nv;
                         } else {
                             for (int r = 0; r < 4 && n + r < g.N; ++r) o[r] = nv[r];
                         }
+                        if (g.row_stats) {
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            if (n + r < g.N) {
-                                st.s1 += nv[r];
-                                st.s2 += (int64_t)nv[r] * nv[r];
+                            for (int r = 0; r < 4; ++r) {
+                                if (n + r < g.N) {
+                                    st.s1 += nv[r];
+                                    st.s2 += (int64_t)nv[r] * nv[r];
+                                }
                             }
                         }
                     }
@@ -807,51 +836,11 @@ __device__ __forceinline__ void gemm32_tile(const GemmArgs &g, const ConvArgs &c
         __syncthreads();
         if constexpr (CONV) {
             if (xblk) {
-                // depthwise conv + squareplus (spec rules 4.3-4.4) down the tile:
                 // thread (cg, run) takes channels ch..ch+3 of staged rows
-                // 3 + 32 run .. (32 rows; the last run 29), as in gemm_tile
+                // 3 + 32 run .. (32 rows; the last run 29)
                 const int run = tid >> 6;
-                const int i0 = 3 + 32 * run, i1 = min(i0 + 32, kG2BM);
-                int gm = m0 + i0;
-                if (gm < g.M) {
-                    int sb = gm / cv.L, t = gm - sb * cv.L;
-                    auto row = [&](int i) { return *reinterpret_cast<const uint32_t *>(&so[g2_ooff(i, 4 * cg)]); };
-                    auto state = [&](int k) -> uint32_t {  // x[k] of sequence sb, k in [-3, -1]
-                        return cv.st_in ? *reinterpret_cast<const uint32_t *>(cv.st_in + ((int64_t)sb * 3 + 3 + k) * cv.D + ch)
-                                        : 0u;
-                    };
-                    uint32_t win[4] = {0, 0, 0, 0};
-                    auto push = [&](uint32_t v) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            win[r] = __builtin_amdgcn_perm(v, win[r], 0x00030201u | ((uint32_t)(4 + r) << 24));
-                    };
-                    for (int j = 3; j >= 1; --j) push(t - j >= 0 ? row(i0 - j) : state(t - j));
-                    for (int i = i0; i < i1 && gm < g.M; ++i, ++gm) {
-                        if (t == 0) {
-                            if (i > i0)
-                                for (int j = 3; j >= 1; --j) push(state(-j));
-                            for (int j = 0; j < 3 - cv.L; ++j)
-                                *reinterpret_cast<uint32_t *>(cv.st_out + ((int64_t)sb * 3 + j) * cv.D + ch) =
-                                    state(cv.L + j - 3);
-                        }
-                        const uint32_t cur = row(i);
-                        push(cur);
-                        uint32_t o = 0;
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int32_t c = __builtin_amdgcn_sdot4((int)win[r], (int)tw[r], tb[r], false);
-                            o |= (uint32_t)(sqp_q(c) & 255) << (8 * r);
-                        }
-                        *reinterpret_cast<uint32_t *>(cv.xs + (int64_t)gm * cv.D + ch) = o;
-                        if (t >= cv.L - 3)
-                            *reinterpret_cast<uint32_t *>(cv.st_out + ((int64_t)sb * 3 + t - (cv.L - 3)) * cv.D + ch) = cur;
-                        if (++t == cv.L) {
-                            t = 0;
-                            ++sb;
-                        }
-                    }
-                }
+                conv_rows(cv, g.M, m0, 3 + 32 * run, min(35 + 32 * run, kG2BM), ch, tw, tb,
+                          [&](int i) { return *reinterpret_cast<const uint32_t *>(&so[g2_ooff(i, 4 * cg)]); });
                 return;
             }
         }
@@ -881,13 +870,14 @@ __device__ __forceinline__ void gemm32_tile(const GemmArgs &g, const ConvArgs &c
             for (int f = 0; f < 2; ++f)
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    v4i nv;
+                    const v4i nv = residual4(g, old[f][c], v4i{acc[f][j][4 * c], acc[f][j][4 * c + 1],
+                                                               acc[f][j][4 * c + 2], acc[f][j][4 * c + 3]});
+                    if (g.row_stats) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int64_t delta = residual_delta(g, acc[f][j][4 * c + i]);
-                        nv[i] = (int32_t)clamp64((int64_t)old[f][c][i] + delta, -kResidualLimit, kResidualLimit);
-                        st.s1 += nv[i];
-                        st.s2 += (int64_t)nv[i] * nv[i];
+                        for (int i = 0; i < 4; ++i) {
+                            st.s1 += nv[i];
+                            st.s2 += (int64_t)nv[i] * nv[i];
+                        }
                     }
                     if (m < g.M)
                         *reinterpret_cast<v4i *>(ob + (int64_t)m * g.ldo + n0 + 64 * wid + 32 * f + 8 * c + 4 * h) = nv;
@@ -913,6 +903,217 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm32_conv_kernel(GemmArgs g,
                                                                                                 ConvArgs cv) {
     gemm32_tile<MI_OUT_INT8, true>(g, cv);
+}
+
+// --------------------------------------------- prefill GEMM, small tiles
+// gemm_ring_kernel: 64 x 64 block tiles, 2 x 2 waves of one 32 x 32 fragment
+// each, for products whose 128 x 128 tiles leave CUs idle or hold one block
+// each.  Such a launch is bound by latency (gemm_kernel's next stage is one
+// memory round trip away, ~1 us a stage), so the tiles are four times as many
+// and the stages come by LDS DMA through a ring of three (36 KB: up to four
+// blocks a CU): a wave waits for its own 3 loads of a stage, a barrier makes
+// every wave's visible and frees the oldest buffer, which is refilled two
+// stages ahead.  MFMA operands, k order and the swizzle of the activation rows
+// are gemm32_kernel's; each wave keeps its own copy of its weight words.  Rings
+// of four and six stages (less blocks a CU) measured 2 to 30% slower, 128 x 64
+// and 64 x 128 tiles 5 to 30%, and eight waves splitting k 5 to 25%.
+// 2000 x 1536 -> 768 RESIDUAL 17.0 -> 9.9 us, 2103 x 2048 -> 1024 20.0 -> 16.1,
+// 100 x 1536 -> 768 15.1 -> 7.2; in_proj with conv, 100 rows of 768 -> 3072
+// 12.2 -> 6.7, 1000 rows 13.1 -> 10.0.
+// Requires K % 128 == 0, N % 32 == 0 (conv: d_inner % 64 == 0), 16-byte aligned
+// a / w with lda % 16 == 0; rows past M and N as in gemm32_kernel.
+constexpr int kRingBM = 64, kRingBN = 64, kRingStages = 3;
+constexpr int kRingConvRows = kRingBM - 3;
+constexpr int kRingOpitch = kRingBN + 16;   // int8 output tile pitch
+
+struct RingSmem {
+    int8_t a[kRingStages][kRingBM * kG2BK];
+    uint32_t w[kRingStages][4][256];   // [stage][wave][lane * 4 + word]
+};
+static_assert(kRingBM * kRingOpitch <= kRingStages * kRingBM * kG2BK, "output tile must fit the ring");
+
+// This wave's LDS reads are done and at most V of its loads are in flight.
+template <int V>
+__device__ __forceinline__ void ring_wait() {
+    __builtin_amdgcn_s_waitcnt((V & 15) | ((V >> 4) << 14) | (7 << 4));   // vmcnt(V) lgkmcnt(0)
+    asm volatile("" ::: "memory");
+}
+
+template <int KIND, bool CONV>
+__device__ __forceinline__ void ring_tile(const GemmArgs &g, const ConvArgs &cv) {
+    constexpr int BN = kRingBN, BM = kRingBM, R = kRingStages;
+    __shared__ __align__(16) RingSmem sm;
+    const int tid = threadIdx.x, lane = tid & 63, wid = wave_id();
+    const int l32 = lane & 31, h = lane >> 5;
+    const int wn = wid & 1, wm = wid >> 1;
+
+    int m0, n0;
+    bool xblk = false;   // block-uniform: a conv x-half tile
+    {
+        auto xcd_run = [](int b, int T) { return (T & 7) == 0 ? (b & 7) * (T >> 3) + (b >> 3) : b; };
+        int t = (int)blockIdx.x, mt, nt;
+        if constexpr (CONV) {
+            const int zb = (int)gridDim.x - cv.x_blocks;
+            t = (cv.x_blocks & 7) == 0 ? (t < cv.x_blocks ? xcd_run(t, cv.x_blocks) : cv.x_blocks + xcd_run(t - cv.x_blocks, zb))
+                                       : t;
+            if (t < cv.x_blocks) {
+                grouped_tile(t, (g.M + kRingConvRows - 1) / kRingConvRows, cv.D / BN, mt, nt);
+                xblk = true;
+                m0 = mt * kRingConvRows - 3;
+                n0 = nt * BN;
+            } else {
+                grouped_tile(t - cv.x_blocks, (g.M + BM - 1) / BM, (g.N - cv.D) / BN, mt, nt);
+                m0 = mt * BM;
+                n0 = cv.D + nt * BN;
+            }
+        } else {
+            grouped_tile(xcd_run(t, (int)gridDim.x), (g.M + BM - 1) / BM, (g.N + BN - 1) / BN, mt, nt);
+            m0 = mt * BM;
+            n0 = nt * BN;
+        }
+    }
+    const int nk = g.K / kG2BK;
+
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t *>(g.a), 0, (int)min((int64_t)g.M * g.lda, (int64_t)INT32_MAX), kBufferRsrcWord3);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t *>(g.w), 0, (int)min((int64_t)g.N * g.kw * 4, (int64_t)INT32_MAX), kBufferRsrcWord3);
+    uint32_t aoffs[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int row = 8 * (2 * wid + j) + (lane >> 3);
+        const int q = (lane & 7) ^ ((row >> 1) & 7);
+        int m = min(m0 + row, g.M - 1);
+        if constexpr (CONV) m = max(m, 0);
+        aoffs[j] = (uint32_t)((int64_t)m * g.lda + 16 * q);
+    }
+    const uint32_t woff = (uint32_t)(((int64_t)min(n0 + 32 * wn + l32, g.N - 1) * g.kw + 4 * h) * 4);
+    auto issue = [&](int kt) {
+        const int b = kt % R;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void_t *)&sm.a[b][(2 * wid + j) * 1024], 16, aoffs[j],
+                                                     (uint32_t)(kt * kG2BK), 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void_t *)&sm.w[b][wid][0], 16, woff,
+                                                 (uint32_t)(kt * (kG2BK / 4)), 0, 0);
+    };
+
+    v16i acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0;
+    int aoff[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) aoff[s] = 32 * wm * kG2BK + g2_aoff(l32, 4 * h + s);
+
+    static_assert(R == 3, "the waits below leave one stage of 3 loads in flight");
+    issue(0);
+    if (nk > 1) issue(1);
+    for (int kt = 0; kt < nk; ++kt) {
+        if (kt + 1 < nk)
+            ring_wait<3>();
+        else
+            ring_wait<0>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (kt + 2 < nk) issue(kt + 2);
+        const int b = kt % R;
+        const v4i wv = *reinterpret_cast<const v4i *>(&sm.w[b][wid][lane * 4]);
+        v4i fa[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) fa[s] = *reinterpret_cast<const v4i *>(&sm.a[b][aoff[s]]);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc = mfma32_i8(unpack16((uint32_t)wv[s]), fa[s], acc);
+    }
+    auto quad = [&](int c) { return v4i{acc[4 * c], acc[4 * c + 1], acc[4 * c + 2], acc[4 * c + 3]}; };
+    // quad(c): features nf + 8 c + 4 h .. + 3, token mf of the tile
+    const int nf = 32 * wn, mf = 32 * wm + l32;
+
+    if constexpr (KIND == MI_OUT_INT8 || KIND == MI_OUT_DECAY_MOD) {
+        int8_t *so = &sm.a[0][0];
+        const int cg = tid & 15, ch = n0 + 4 * cg;
+        uint32_t tw[4] = {0, 0, 0, 0};
+        int32_t tb[4] = {0, 0, 0, 0};
+        if constexpr (CONV) {
+            if (xblk) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    tw[r] = *reinterpret_cast<const uint32_t *>(cv.w + (int64_t)(ch + r) * 4);
+                    tb[r] = cv.b[ch + r];
+                }
+            }
+        }
+        __syncthreads();   // every wave is done reading the ring (no loads are in flight)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const v4i v = quad(c);
+            uint32_t pk = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int q = rshr32(v[i], g.shift);
+                pk |= (uint32_t)((KIND == MI_OUT_INT8 ? clamp32(q, -127, 127) : clamp32(q, -20, 20)) & 255) << (8 * i);
+            }
+            *reinterpret_cast<uint32_t *>(&so[mf * kRingOpitch + nf + 8 * c + 4 * h]) = pk;
+        }
+        __syncthreads();
+        if constexpr (CONV) {
+            if (xblk) {
+                // thread (cg, run): channels ch..ch+3 of staged rows 3 + 4 run .. (4 rows; the last run 1)
+                const int i0 = 3 + 4 * (tid >> 4);
+                conv_rows(cv, g.M, m0, i0, min(i0 + 4, BM), ch, tw, tb,
+                          [&](int i) { return *reinterpret_cast<const uint32_t *>(&so[i * kRingOpitch + 4 * cg]); });
+                return;
+            }
+        }
+        // thread t stores 16-byte granule t % 4 of row t / 4
+        const int row = tid >> 2, gr = tid & 3, gm = m0 + row, gn = n0 + 16 * gr;
+        if (gm < g.M && gn < g.N)
+            *reinterpret_cast<v4i *>((int8_t *)g.out + (int64_t)gm * g.ldo + gn) =
+                *reinterpret_cast<const v4i *>(&so[row * kRingOpitch + 16 * gr]);
+    } else if (n0 + nf < g.N) {   // N % 32 == 0: a wave's features are all stored or none
+        const int m = m0 + mf, n = n0 + nf + 4 * h;
+        if constexpr (KIND == MI_OUT_RESIDUAL) {
+            int32_t *o = (int32_t *)g.out + (int64_t)min(m, g.M - 1) * g.ldo + n;
+            v4i old[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) old[c] = *reinterpret_cast<const v4i *>(o + 8 * c);
+            RowStat st{0, 0};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const v4i nv = residual4(g, old[c], quad(c));
+                if (g.row_stats) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        st.s1 += nv[i];
+                        st.s2 += (int64_t)nv[i] * nv[i];
+                    }
+                }
+                if (m < g.M) *reinterpret_cast<v4i *>(o + 8 * c) = nv;
+            }
+            if (g.row_stats) {
+                st.s1 += __shfl_xor(st.s1, 32);
+                st.s2 += __shfl_xor(st.s2, 32);
+                if (h == 0 && m < g.M) {
+                    atomicAdd(reinterpret_cast<unsigned long long *>(g.row_stats + 2 * (int64_t)m), (unsigned long long)st.s1);
+                    atomicAdd(reinterpret_cast<unsigned long long *>(g.row_stats + 2 * (int64_t)m + 1),
+                              (unsigned long long)st.s2);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) store4<KIND>(g, m, n + 8 * c, quad(c));
+        }
+    }
+}
+
+template <int KIND>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void gemm_ring_kernel(GemmArgs g) {
+    ring_tile<KIND, false>(g, ConvArgs{});
+}
+
+// in_proj (int8 out, shifted) with the conv + squareplus of the x half fused
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void gemm_ring_conv_kernel(GemmArgs g,
+                                                                                                   ConvArgs cv) {
+    ring_tile<MI_OUT_INT8, true>(g, cv);
 }
 
 // gemm_any_kernel: any k % 16 == 0 and 4-byte aligned weights (e.g. dt_proj
@@ -1588,6 +1789,10 @@ GemmArgs make_args(const int8_t *a, int lda, const uint8_t *w, void *out, int ld
     g.lda = lda; g.ldo = ldo; g.M = m; g.N = n; g.K = k; g.kw = k / 16;
     g.shift = shift; g.res_mult = res_mult; g.res_shift = res_shift; g.w_scale = w_scale; g.row_stats = row_stats;
     g.res_clamp = res_clamp > 0 ? res_clamp : INT32_MAX;
+    // |acc| <= 128 * 2 * k (the widest code of a packed weight is -2); the
+    // shifted product plus rounding stays below 2^31
+    const int64_t bound = std::min<int64_t>((int64_t)256 * k, g.res_clamp) * std::abs((int64_t)res_mult);
+    g.res32 = res_shift >= 1 && res_shift <= 31 && (int64_t)256 * k <= INT32_MAX && (bound >> res_shift) < INT32_MAX - 1;
     return g;
 }
 
@@ -1601,6 +1806,20 @@ bool gemm32_fits(const GemmArgs &g, int64_t tiles) {
     return g.K > 0 && g.K % kG2BK == 0 && g.N % kG2BN == 0 && g.M > 64 && aligned(g.a, 16) && g.lda % 16 == 0 &&
            aligned(g.w, 16) && (int64_t)g.M * g.lda <= INT32_MAX && (int64_t)g.N * g.kw * 4 <= INT32_MAX &&
            tiles >= kG2MinTiles;
+}
+
+// Shapes and layouts gemm_ring_kernel takes, where its 64 x 64 tiles are few
+// enough.  Up to two a CU it always won (4096 deep, 512 tiles: 30.2 -> 18.7
+// us); beyond that the larger tiles' fewer LDS bytes an operation count, the
+// sooner the deeper k: 768 deep 1152 tiles 16.1 -> 13.4 us but 1560 tiles with
+// conv 14.4 -> 15.4; 1536 deep 1020 tiles 22.6 -> 18.1, 1536 tiles 25.1 ->
+// 24.9; 2048 deep 528 tiles 20.0 -> 16.1, 784 tiles 15.0 -> 16.6; 4096 deep
+// 1024 tiles 32.9 -> 33.7.
+constexpr int64_t kRingMaxTiles = 1152, kRingMaxWork = 1024 * 1536;
+bool ring_fits(const GemmArgs &g, int64_t tiles) {
+    return g.K > 0 && g.K % kG2BK == 0 && g.N % 32 == 0 && aligned(g.a, 16) && g.lda % 16 == 0 && aligned(g.w, 16) &&
+           (int64_t)g.M * g.lda <= INT32_MAX && (int64_t)g.N * g.kw * 4 <= INT32_MAX &&
+           (tiles <= 512 || (tiles <= kRingMaxTiles && tiles * g.K <= kRingMaxWork));
 }
 
 template <int KIND>
@@ -1618,6 +1837,12 @@ hipError_t launch_gemm_kind(const GemmArgs &g, hipStream_t st) {
                                dim3(256), 0, st, g);
             return hipGetLastError();
         }
+    }
+    const int64_t ring = (int64_t)((g.M + kRingBM - 1) / kRingBM) * ((g.N + kRingBN - 1) / kRingBN);
+    const int out_unit = kInt8Out ? 16 : 4;
+    if (ring_fits(g, ring) && g.ldo % out_unit == 0 && aligned(g.out, 16)) {
+        hipLaunchKernelGGL(gemm_ring_kernel<KIND>, dim3((unsigned)ring), dim3(256), 0, st, g);
+        return hipGetLastError();
     }
     if constexpr (KIND == MI_OUT_INT8 || KIND == MI_OUT_RESIDUAL) {
         const bool out_ok = KIND == MI_OUT_INT8 ? g.ldo % 16 == 0 && aligned(g.out, 16)
@@ -1828,17 +2053,23 @@ extern "C" mi_status mi_in_proj_conv(const int8_t *a, int lda, const uint8_t *w_
     ConvArgs cv{};
     cv.w = conv_w; cv.b = conv_b; cv.st_in = state_in; cv.st_out = state_out; cv.xs = xs;
     cv.D = d_inner; cv.L = len;
+    const int64_t ring = (int64_t)((m + kRingConvRows - 1) / kRingConvRows + (m + kRingBM - 1) / kRingBM) * (d_inner / kRingBN);
+    const bool small = ring_fits(g, ring);
     const int64_t tiles32 = (int64_t)((m + kG2ConvRows - 1) / kG2ConvRows + (m + kG2BM - 1) / kG2BM) * (d_inner / kG2BN);
-    const bool big = d_inner % kG2BN == 0 && gemm32_fits(g, tiles32);
-    const int64_t nt = d_inner / (big ? kG2BN : kBN);
-    const int64_t xb = (int64_t)((m + (big ? kG2ConvRows : kConvRows) - 1) / (big ? kG2ConvRows : kConvRows)) * nt;
-    const int64_t zb = (int64_t)((m + kBM - 1) / kBM) * nt;   // kG2BM == kBM
+    const bool big = !small && d_inner % kG2BN == 0 && gemm32_fits(g, tiles32);
+    const int64_t nt = d_inner / (small ? kRingBN : big ? kG2BN : kBN);
+    const int rows = small ? kRingConvRows : kConvRows, zrows = small ? kRingBM : kBM;   // kG2BM == kBM
+    const int64_t xb = (int64_t)((m + rows - 1) / rows) * nt;
+    const int64_t zb = (int64_t)((m + zrows - 1) / zrows) * nt;
     MI_REQUIRE(xb + zb <= INT32_MAX, MI_ERR_BAD_DIM, "%s: grid too large", fn);
     cv.x_blocks = (int)xb;
-    if (big)
-        hipLaunchKernelGGL(gemm32_conv_kernel, dim3((unsigned)(xb + zb)), dim3(256), 0, as_stream(stream), g, cv);
+    const dim3 grid((unsigned)(xb + zb));
+    if (small)
+        hipLaunchKernelGGL(gemm_ring_conv_kernel, grid, dim3(256), 0, as_stream(stream), g, cv);
+    else if (big)
+        hipLaunchKernelGGL(gemm32_conv_kernel, grid, dim3(256), 0, as_stream(stream), g, cv);
     else
-        hipLaunchKernelGGL(gemm_conv_kernel, dim3((unsigned)(xb + zb)), dim3(256), 0, as_stream(stream), g, cv);
+        hipLaunchKernelGGL(gemm_conv_kernel, grid, dim3(256), 0, as_stream(stream), g, cv);
     return check_launch(fn);
 }
 
