@@ -90,6 +90,16 @@ __device__ __forceinline__ v4i residual4(const GemmArgs &g, v4i old, v4i acc) {
     return nv;
 }
 
+// INT8 / DECAY_MOD outputs of 4 consecutive features as one dword.
+template <int KIND>
+__device__ __forceinline__ uint32_t requant4(const GemmArgs &g, v4i acc) {
+    constexpr int kLim = KIND == MI_OUT_INT8 ? 127 : 20;
+    int v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = clamp32(rshr32(acc[r], g.shift), -kLim, kLim);
+    return pack4(v[0], v[1], v[2], v[3]);
+}
+
 // FLOAT outputs of features n .. n + 3: fp32(acc) * (w_scale * x_scale[m]) (rational_bitnet.py:208),
 // then the bias (rational_bitnet.py:211-213); features past N repeat the last one's bias, unstored.
 __device__ __forceinline__ v4f float_out(const GemmArgs &g, float x_scale, int n, v4i acc) {
@@ -114,16 +124,11 @@ __device__ __forceinline__ RowStat store4(const GemmArgs &g, int m, int n, v4i a
     const bool full = n + 3 < g.N;
     if constexpr (KIND == MI_OUT_INT8 || KIND == MI_OUT_DECAY_MOD) {
         int8_t *o = (int8_t *)g.out + (int64_t)m * g.ldo + n;
-        int v[4];
-        for (int r = 0; r < 4; ++r) {
-            int q = rshr32(acc[r], g.shift);
-            v[r] = KIND == MI_OUT_INT8 ? clamp32(q, -127, 127) : clamp32(q, -20, 20);
-        }
+        const uint32_t pk = requant4<KIND>(g, acc);
         if (full) {
-            *reinterpret_cast<uint32_t *>(o) = (uint32_t)(v[0] & 255) | ((uint32_t)(v[1] & 255) << 8) |
-                                               ((uint32_t)(v[2] & 255) << 16) | ((uint32_t)(v[3] & 255) << 24);
+            *reinterpret_cast<uint32_t *>(o) = pk;
         } else {
-            for (int r = 0; r < 4 && n + r < g.N; ++r) o[r] = (int8_t)v[r];
+            for (int r = 0; r < 4 && n + r < g.N; ++r) o[r] = (int8_t)(pk >> (8 * r));
         }
     } else if constexpr (KIND == MI_OUT_INT32) {
         int32_t *o = (int32_t *)g.out + (int64_t)m * g.ldo + n;
@@ -251,12 +256,10 @@ __device__ __forceinline__ void conv_rows(const ConvArgs &cv, int M, int m0, int
         }
         const uint32_t cur = row(i);
         push(cur);
-        uint32_t o = 0;
+        int32_t c[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int32_t c = __builtin_amdgcn_sdot4((int)win[r], (int)tw[r], tb[r], false);
-            o |= (uint32_t)(sqp_q(c) & 255) << (8 * r);
-        }
+        for (int r = 0; r < 4; ++r) c[r] = __builtin_amdgcn_sdot4((int)win[r], (int)tw[r], tb[r], false);
+        const uint32_t o = sqp4(c[0], c[1], c[2], c[3]);
         *reinterpret_cast<uint32_t *>(cv.xs + (int64_t)gm * cv.D + ch) = o;
         if (t >= cv.L - 3)
             *reinterpret_cast<uint32_t *>(cv.st_out + ((int64_t)sb * 3 + t - (cv.L - 3)) * cv.D + ch) = cur;
@@ -447,13 +450,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const ConvArgs &cv)
         for (int j = 0; j < MJ; ++j)
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
-                uint32_t pk = 0;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int q = rshr32(acc[i][j][r], g.shift);
-                    const int v = KIND == MI_OUT_INT8 ? clamp32(q, -127, 127) : clamp32(q, -20, 20);
-                    pk |= (uint32_t)(v & 255) << (8 * r);
-                }
+                const uint32_t pk = requant4<KIND>(g, acc[i][j]);
                 *reinterpret_cast<uint32_t *>(&sO[(mb + j * 16 + l16) * kOpitch + nb + i * 16 + 4 * lq]) = pk;
             }
         __syncthreads();
@@ -825,12 +822,8 @@ __device__ __forceinline__ void gemm32_tile(const GemmArgs &g, const ConvArgs &c
             for (int j = 0; j < 4; ++j)
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    uint32_t pk = 0;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int q = rshr32(acc[f][j][4 * c + i], g.shift);
-                        pk |= (uint32_t)(clamp32(q, -127, 127) & 255) << (8 * i);
-                    }
+                    const uint32_t pk = requant4<KIND>(g, v4i{acc[f][j][4 * c], acc[f][j][4 * c + 1],
+                                                              acc[f][j][4 * c + 2], acc[f][j][4 * c + 3]});
                     *reinterpret_cast<uint32_t *>(&so[g2_ooff(32 * j + l32, 64 * wid + 32 * f + 8 * c + 4 * h)]) = pk;
                 }
         __syncthreads();
@@ -1045,14 +1038,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs &g, const ConvArgs &cv)
         __syncthreads();   // every wave is done reading the ring (no loads are in flight)
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const v4i v = quad(c);
-            uint32_t pk = 0;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int q = rshr32(v[i], g.shift);
-                pk |= (uint32_t)((KIND == MI_OUT_INT8 ? clamp32(q, -127, 127) : clamp32(q, -20, 20)) & 255) << (8 * i);
-            }
-            *reinterpret_cast<uint32_t *>(&so[mf * kRingOpitch + nf + 8 * c + 4 * h]) = pk;
+            *reinterpret_cast<uint32_t *>(&so[mf * kRingOpitch + nf + 8 * c + 4 * h]) = requant4<KIND>(g, quad(c));
         }
         __syncthreads();
         if constexpr (CONV) {

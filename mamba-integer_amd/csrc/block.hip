@@ -365,15 +365,16 @@ __global__ __launch_bounds__(256) void conv_sqp_kernel(const int8_t *xz, int64_t
     uint32_t keep_state[3] = {win[0], win[1], win[2]};  // x[-3..-1] for the state update when L < 3
     for (int t = t0; t < t1; ++t) {
         const uint32_t cur = xrow(t);
-        uint32_t o = 0;
+        int32_t s4[4];
         for (int c = 0; c < 4; ++c) {
             int32_t acc = bv[c];
             acc += wv[c][0] * (int)(int8_t)(win[0] >> (8 * c));
             acc += wv[c][1] * (int)(int8_t)(win[1] >> (8 * c));
             acc += wv[c][2] * (int)(int8_t)(win[2] >> (8 * c));
             acc += wv[c][3] * (int)(int8_t)(cur >> (8 * c));
-            o |= (uint32_t)(sqp_q(acc) & 255) << (8 * c);
+            s4[c] = acc;
         }
+        const uint32_t o = sqp4(s4[0], s4[1], s4[2], s4[3]);
         *reinterpret_cast<uint32_t *>(xs + ((int64_t)b * L + t) * D + d) = o;
         win[0] = win[1];
         win[1] = win[2];

@@ -389,7 +389,7 @@ __global__ __launch_bounds__(256) void norm_gemv_kernel(NormGemvArgs g0) {
         if (ok) {
             const int32_t c = ecb + (int)(int8_t)ecw * ecs0 + (int)(int8_t)(ecw >> 8) * ecs1 +
                               (int)(int8_t)(ecw >> 16) * ecs2 + (int)(int8_t)(ecw >> 24) * q;
-            xsv = sqp_q(c);
+            xsv = sqp1(c);
             g.xs[(int64_t)m * g.conv_d + fe] = (int8_t)xsv;
             int8_t *st = g.conv_state + (int64_t)m * 3 * g.conv_d + fe;
             st[0] = (int8_t)ecs1;
@@ -470,18 +470,19 @@ __global__ __launch_bounds__(256) void norm_gemv_kernel(NormGemvArgs g0) {
         for (int r = 0; r < 4; ++r) v[r] = clamp32(rshr32(acc[r], g.shift), -127, 127);
         if (conv) {
             // depthwise conv step (conv1d_step.cu:30-57) + squareplus on 4 channels
-            uint32_t xsw = 0, cur = 0;
+            uint32_t cur = 0;
+            int32_t c4[4];
             for (int r = 0; r < 4; ++r) {
                 int32_t c = cb[r];
                 c += (int)(int8_t)(cw[r]) * (int)(int8_t)(cs0 >> (8 * r));
                 c += (int)(int8_t)(cw[r] >> 8) * (int)(int8_t)(cs1 >> (8 * r));
                 c += (int)(int8_t)(cw[r] >> 16) * (int)(int8_t)(cs2 >> (8 * r));
                 c += (int)(int8_t)(cw[r] >> 24) * v[r];
-                xsw |= (uint32_t)(sqp_q(c) & 255) << (8 * r);
+                c4[r] = c;
                 cur |= (uint32_t)(v[r] & 255) << (8 * r);
             }
             int8_t *st = g.conv_state + (int64_t)m * 3 * g.conv_d;
-            *reinterpret_cast<uint32_t *>(g.xs + (int64_t)m * g.conv_d + nf) = xsw;
+            *reinterpret_cast<uint32_t *>(g.xs + (int64_t)m * g.conv_d + nf) = sqp4(c4[0], c4[1], c4[2], c4[3]);
             *reinterpret_cast<uint32_t *>(st + nf) = cs1;
             *reinterpret_cast<uint32_t *>(st + g.conv_d + nf) = cs2;
             *reinterpret_cast<uint32_t *>(st + 2 * g.conv_d + nf) = cur;
@@ -1502,16 +1503,16 @@ __global__ __launch_bounds__(64 * kConvXWaves) void conv_step_xproj_kernel(ConvX
         const uint32_t s2 = *reinterpret_cast<const uint32_t *>(st + 2 * g.D + ch);
         const v4i cw = *reinterpret_cast<const v4i *>(g.conv_w + (int64_t)ch * 4);
         const v4i cb = *reinterpret_cast<const v4i *>(g.conv_b + ch);
-        uint32_t o = 0;
+        int32_t c4[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const uint32_t w = (uint32_t)cw[e];
-            const int32_t acc = cb[e] + (int)(int8_t)w * (int)(int8_t)(s0 >> (8 * e)) +
+            c4[e] = cb[e] + (int)(int8_t)w * (int)(int8_t)(s0 >> (8 * e)) +
                                 (int)(int8_t)(w >> 8) * (int)(int8_t)(s1 >> (8 * e)) +
                                 (int)(int8_t)(w >> 16) * (int)(int8_t)(s2 >> (8 * e)) +
                                 (int)(int8_t)(w >> 24) * (int)(int8_t)(x >> (8 * e));
-            o |= (uint32_t)(sqp_q(acc) & 255) << (8 * e);
         }
+        const uint32_t o = sqp4(c4[0], c4[1], c4[2], c4[3]);
         *reinterpret_cast<uint32_t *>(g.xs + (int64_t)m * g.D + ch) = o;
         *reinterpret_cast<uint32_t *>(st + ch) = s1;
         *reinterpret_cast<uint32_t *>(st + g.D + ch) = s2;
@@ -1609,16 +1610,16 @@ __global__ __launch_bounds__(256) void conv_step_xpart_kernel(ConvXArgs g) {
     };
     // depthwise conv step (conv1d_step.cu:30-57) + squareplus of 4 channels
     auto conv_finish = [&](const ConvIn &c, int ch) {
-        uint32_t o = 0;
+        int32_t c4[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const uint32_t w = (uint32_t)c.cw[e];
-            const int32_t acc = c.cb[e] + (int)(int8_t)w * (int)(int8_t)(c.s0 >> (8 * e)) +
+            c4[e] = c.cb[e] + (int)(int8_t)w * (int)(int8_t)(c.s0 >> (8 * e)) +
                                 (int)(int8_t)(w >> 8) * (int)(int8_t)(c.s1 >> (8 * e)) +
                                 (int)(int8_t)(w >> 16) * (int)(int8_t)(c.s2 >> (8 * e)) +
                                 (int)(int8_t)(w >> 24) * (int)(int8_t)(c.x >> (8 * e));
-            o |= (uint32_t)(sqp_q(acc) & 255) << (8 * e);
         }
+        const uint32_t o = sqp4(c4[0], c4[1], c4[2], c4[3]);
         *reinterpret_cast<uint32_t *>(xso + ch) = o;
         *reinterpret_cast<uint32_t *>(st + ch) = c.s1;
         *reinterpret_cast<uint32_t *>(st + g.D + ch) = c.s2;
