@@ -1102,6 +1102,43 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void g
     ring_tile<MI_OUT_INT8, true>(g, cv);
 }
 
+// gemm_k64_kernel: k <= 64 (dt_proj), int8 outputs in whole 16-byte groups.
+// One MFMA deep, so it is bound by its output's stores and by latency:
+// nothing goes through LDS.  A wave owns 64 features x 64 tokens.  Row 4 i + r
+// of its weight fragment f is feature 16 i + 4 f + r, so the four fragments'
+// results of a lane (group lq: rows 4 lq ..) are the 16 consecutive features
+// 16 lq .. of its token, one 16-byte store.  All loads are unconditional from
+// clamped addresses and issued before the first product; words past k are
+// zeroed.  @@
+template <int KIND>
+__global__ __launch_bounds__(256) void gemm_k64_kernel(GemmArgs g) {
+    const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
+    const int ntiles = (g.N + 255) / 256;
+    const int n0 = 256 * ((int)blockIdx.x % ntiles) + 64 * wave_id(), m0 = 64 * ((int)blockIdx.x / ntiles);
+    if (n0 >= g.N) return;
+    const int lw = min(lq, g.kw - 1);
+    v4i fa[4];
+    uint32_t w[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+        fa[t] = *reinterpret_cast<const v4i *>(g.a + (int64_t)min(m0 + 16 * t + l16, g.M - 1) * g.lda + 16 * lw);
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+        w[f] = g.w[(int64_t)min(n0 + 16 * (l16 >> 2) + 4 * f + (l16 & 3), g.N - 1) * g.kw + lw];
+    v4i fw[4];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) fw[f] = unpack16(lq < g.kw ? w[f] : 0u);
+    const int n = n0 + 16 * lq;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        v4i o;
+#pragma unroll
+        for (int f = 0; f < 4; ++f) o[f] = (int)requant4<KIND>(g, mfma_i8(fw[f], fa[t], v4i{0, 0, 0, 0}));
+        const int m = m0 + 16 * t + l16;
+        if (m < g.M && n < g.N) *reinterpret_cast<v4i *>((int8_t *)g.out + (int64_t)m * g.ldo + n) = o;
+    }
+}
+
 // gemm_any_kernel: any k % 16 == 0 and 4-byte aligned weights (e.g. dt_proj
 // with k = dt_rank): 4 waves of 64x64, weights fetched one word per thread.
 // 64-deep halves of a stage that lie wholly past K are skipped (k = 48 has
@@ -1193,13 +1230,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void g
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                uint32_t pk = 0;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int q = rshr32(acc[i][j][r], g.shift);
-                    const int v = KIND == MI_OUT_INT8 ? clamp32(q, -127, 127) : clamp32(q, -20, 20);
-                    pk |= (uint32_t)(v & 255) << (8 * r);
-                }
+                const uint32_t pk = requant4<KIND>(g, acc[i][j]);
                 *reinterpret_cast<uint32_t *>(&sO[(wm * 64 + j * 16 + l16) * kOpitch + wn * 64 + i * 16 + 4 * lq]) = pk;
             }
         __syncthreads();
@@ -1435,34 +1466,34 @@ __global__ __launch_bounds__(64 * WAVES) void gemv64_kernel(GemmArgs g) {
 // bank groups.  Same chunk ownership and results as gemv64_kernel.
 constexpr int kG64Waves = 4, kG64U = 2;
 
-// Blocks along y take 64-row groups (rows [64y, 64y + 64)): the prefill form
-// for few outputs (x_proj, N <= 160, FT = 5), where 128 x 128 GEMM tiles would
-// leave most CUs idle.
-template <int KIND, int FT>
+// Blocks along y take groups of 16 TT rows (TT = 4 in a decode step): the
+// prefill form for few outputs (x_proj, N <= 160, FT = 5), where 128 x 128 GEMM
+// tiles would leave most CUs idle.
+template <int KIND, int FT, int TT>
 __global__ __launch_bounds__(64 * kG64Waves) void gemv64s_kernel(GemmArgs g) {
     constexpr int WAVES = kG64Waves, U = kG64U;
     if (gridDim.y > 1) {
         constexpr int kOutBytes = KIND == MI_OUT_INT8 || KIND == MI_OUT_DECAY_MOD ? 1 : 4;
-        const int64_t m0 = 64 * (int64_t)blockIdx.y;
+        const int64_t m0 = 16 * TT * (int64_t)blockIdx.y;
         g.a += m0 * g.lda;
         g.out = (char *)g.out + m0 * g.ldo * kOutBytes;
         if (g.x_scale) g.x_scale += m0;
         if (g.row_stats) g.row_stats += 2 * m0;
-        g.M = min(64, g.M - (int)m0);
+        g.M = min(16 * TT, g.M - (int)m0);
     }
-    __shared__ __align__(16) int8_t stage[WAVES][U][64 * 256];
-    static_assert(FT * 4 * 64 * 16 <= U * 64 * 256, "partial sums reuse the wave's staging region");
+    __shared__ __align__(16) int8_t stage[WAVES][U][16 * TT * 256];
+    static_assert(FT * TT * 64 * 16 <= U * 16 * TT * 256, "partial sums reuse the wave's staging region");
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), l16 = lane & 15, lq = lane >> 4;
     const int n0 = blockIdx.x * 16 * FT;
     const int nchunk = g.kw / 16;
     const uint32_t *wrow[FT];
 #pragma unroll
     for (int f = 0; f < FT; ++f) wrow[f] = g.w + (int64_t)min(n0 + 16 * f + l16, g.N - 1) * g.kw;
-    v4i acc[FT][4];
+    v4i acc[FT][TT];
 #pragma unroll
     for (int f = 0; f < FT; ++f)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[f][t] = v4i{0, 0, 0, 0};
+        for (int t = 0; t < TT; ++t) acc[f][t] = v4i{0, 0, 0, 0};
     // this lane's row and segment in each 4-row load (rows past M read row M - 1)
     const int srow = lane >> 4;
     for (int c0 = wave; c0 < nchunk; c0 += U * WAVES) {
@@ -1473,7 +1504,7 @@ __global__ __launch_bounds__(64 * kG64Waves) void gemv64s_kernel(GemmArgs g) {
 #pragma unroll
             for (int f = 0; f < FT; ++f) wv[u][f] = *reinterpret_cast<const v4i *>(wrow[f] + 16 * c + 4 * lq);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
+            for (int r = 0; r < 4 * TT; ++r) {
                 const int row = 4 * r + srow;
                 const int seg = (lane & 15) ^ (row & 15);
                 const int8_t *src = g.a + (int64_t)min(row, g.M - 1) * g.lda + 256 * c + 16 * seg;
@@ -1488,16 +1519,16 @@ __global__ __launch_bounds__(64 * kG64Waves) void gemv64s_kernel(GemmArgs g) {
             if (c0 + WAVES * u < nchunk) {  // same for the whole wave
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    v4i xv[4];
+                    v4i xv[TT];
 #pragma unroll
-                    for (int t = 0; t < 4; ++t)
+                    for (int t = 0; t < TT; ++t)
                         xv[t] = *reinterpret_cast<const v4i *>(
                             &stage[wave][u][(16 * t + l16) * 256 + 16 * ((4 * lq + j) ^ l16)]);
 #pragma unroll
                     for (int f = 0; f < FT; ++f) {
                         const v4i fw = unpack16((uint32_t)wv[u][f][j]);
 #pragma unroll
-                        for (int t = 0; t < 4; ++t) acc[f][t] = mfma_i8(fw, xv[t], acc[f][t]);
+                        for (int t = 0; t < TT; ++t) acc[f][t] = mfma_i8(fw, xv[t], acc[f][t]);
                     }
                 }
             }
@@ -1506,20 +1537,22 @@ __global__ __launch_bounds__(64 * kG64Waves) void gemv64s_kernel(GemmArgs g) {
         __builtin_amdgcn_wave_barrier();
     }
     // partial sums into the wave's own region, then waves 0-3 add them up for one token tile each
-    v4i *part = reinterpret_cast<v4i *>(&stage[wave][0][0]);   // [FT][4][64]
+    v4i *part = reinterpret_cast<v4i *>(&stage[wave][0][0]);   // [FT][TT][64]
 #pragma unroll
     for (int f = 0; f < FT; ++f)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) part[(f * 4 + t) * 64 + lane] = acc[f][t];
+        for (int t = 0; t < TT; ++t) part[(f * TT + t) * 64 + lane] = acc[f][t];
     __syncthreads();
-    const int m = 16 * wave + l16;
+    // wave w finishes the 16 x 16 tiles w, w + 4, ... (feature tile i / TT, token tile i % TT)
 #pragma unroll
-    for (int f = 0; f < FT; ++f) {
+    for (int i0 = 0; i0 < FT * TT; i0 += WAVES) {
+        const int i = i0 + wave;
+        if (i >= FT * TT) break;
         v4i v = v4i{0, 0, 0, 0};
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w)
-            v += reinterpret_cast<const v4i *>(&stage[w][0][0])[(f * 4 + wave) * 64 + lane];
-        const RowStat st = store4<KIND>(g, m, n0 + 16 * f + 4 * lq, v);
+        for (int w = 0; w < WAVES; ++w) v += reinterpret_cast<const v4i *>(&stage[w][0][0])[i * 64 + lane];
+        const int m = 16 * (i % TT) + l16;
+        const RowStat st = store4<KIND>(g, m, n0 + 16 * (i / TT) + 4 * lq, v);
         if (KIND == MI_OUT_RESIDUAL && g.row_stats) flush_row_stat(g, st, m, lq);
     }
 }
@@ -1801,6 +1834,7 @@ bool gemm32_fits(const GemmArgs &g, int64_t tiles) {
 // conv 14.4 -> 15.4; 1536 deep 1020 tiles 22.6 -> 18.1, 1536 tiles 25.1 ->
 // 24.9; 2048 deep 528 tiles 20.0 -> 16.1, 784 tiles 15.0 -> 16.6; 4096 deep
 // 1024 tiles 32.9 -> 33.7.
+constexpr int kCus = 256;
 constexpr int64_t kRingMaxTiles = 1152, kRingMaxWork = 1024 * 1536;
 bool ring_fits(const GemmArgs &g, int64_t tiles) {
     return g.K > 0 && g.K % kG2BK == 0 && g.N % 32 == 0 && aligned(g.a, 16) && g.lda % 16 == 0 && aligned(g.w, 16) &&
@@ -1813,15 +1847,34 @@ hipError_t launch_gemm_kind(const GemmArgs &g, hipStream_t st) {
     const dim3 grid((unsigned)(((g.M + kBM - 1) / kBM) * ((g.N + kBN - 1) / kBN)));
     constexpr bool kInt8Out = KIND == MI_OUT_INT8 || KIND == MI_OUT_DECAY_MOD;
     if constexpr (kInt8Out || KIND == MI_OUT_INT32) {
-        // few outputs (x_proj): 80 features x 64 rows per block, so each
-        // 64-row activation slab is read once per 80 outputs and every CU is
+        // few outputs (x_proj): 80 features x 16, 32 or 64 rows per block, so
+        // each activation row is read once per 80 outputs and the CUs are
         // busy (x_proj at d768, 16384 x 1536 -> 80: 12.5 -> 9.2 us; at K = 4096
-        // the GEMM tiles stay faster: 43 vs 70 us)
+        // the GEMM tiles stay faster: 43 vs 70 us).  A block's time is mostly
+        // its loads', which grow with its rows: the fewest rows that fit one
+        // block per CU (2000 rows 8.5 us with 64, 6.6 with 32, 5.6 with 16;
+        // 6000 rows 8.7, 6.8, 7.3; 16384 rows 8.8, 9.4, 10.5), and past that
+        // 32 (32768 rows 19.2, 16.4, 17.3; 64-row blocks run one a CU)
         if (g.N <= 160 && g.M > 64 && (g.M + 63) / 64 <= 65535 && g.kw % 16 == 0 && g.kw / 16 <= 8 &&
             aligned(g.w, 16) && aligned(g.a, 16) && g.lda % 16 == 0) {
-            hipLaunchKernelGGL((gemv64s_kernel<KIND, 5>), dim3((unsigned)((g.N + 79) / 80), (unsigned)((g.M + 63) / 64)),
-                               dim3(256), 0, st, g);
+            const int cols = (g.N + 79) / 80;
+            auto rows = [&](int r) { return (g.M + r - 1) / r; };
+            if (cols * rows(16) <= kCus)
+                hipLaunchKernelGGL((gemv64s_kernel<KIND, 5, 1>), dim3((unsigned)cols, (unsigned)rows(16)), dim3(256), 0, st, g);
+            else if (cols * rows(32) <= kCus || (cols * rows(64) > kCus && rows(32) <= 65535))
+                hipLaunchKernelGGL((gemv64s_kernel<KIND, 5, 2>), dim3((unsigned)cols, (unsigned)rows(32)), dim3(256), 0, st, g);
+            else
+                hipLaunchKernelGGL((gemv64s_kernel<KIND, 5, 4>), dim3((unsigned)cols, (unsigned)rows(64)), dim3(256), 0, st, g);
             return hipGetLastError();
+        }
+    }
+    if constexpr (kInt8Out) {
+        if (g.K > 0 && g.K <= 64 && g.N % 16 == 0 && g.ldo % 16 == 0 && aligned(g.out, 16)) {
+            const int64_t blocks = (int64_t)((g.M + 63) / 64) * ((g.N + 255) / 256);
+            if (blocks <= INT32_MAX) {
+                hipLaunchKernelGGL(gemm_k64_kernel<KIND>, dim3((unsigned)blocks), dim3(256), 0, st, g);
+                return hipGetLastError();
+            }
         }
     }
     const int64_t ring = (int64_t)((g.M + kRingBM - 1) / kRingBM) * ((g.N + kRingBN - 1) / kRingBN);
@@ -1892,7 +1945,7 @@ hipError_t launch_gemv_kind(const GemmArgs &g, hipStream_t st) {
         // (many 16-word chunks per block) spreads over 8 or 16 waves
         const int nchunk = g.kw / 16;
         if ((g.N + 31) / 32 >= 128 && nchunk <= 8)
-            hipLaunchKernelGGL((gemv64s_kernel<KIND, 2>), dim3((unsigned)((g.N + 31) / 32)), dim3(256), 0, st, g);
+            hipLaunchKernelGGL((gemv64s_kernel<KIND, 2, 4>), dim3((unsigned)((g.N + 31) / 32)), dim3(256), 0, st, g);
         else if (nchunk <= 8)
             hipLaunchKernelGGL((gemv64_kernel<KIND, 1, 4>), dim3((unsigned)((g.N + 15) / 16)), dim3(256), 0, st, g);
         else if (nchunk <= 16)
