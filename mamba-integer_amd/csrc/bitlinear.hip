@@ -1109,7 +1109,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void g
 // results of a lane (group lq: rows 4 lq ..) are the 16 consecutive features
 // 16 lq .. of its token, one 16-byte store.  All loads are unconditional from
 // clamped addresses and issued before the first product; words past k are
-// zeroed.  @@
+// zeroed.  Against gemm_any_kernel's 128 x 128 tiles through LDS: 2000 x 48 ->
+// 1536 5.2 -> 4.3 us, 16384 x 48 -> 1536 13.3 -> 10.7 (26 MB: 2.5 TB/s).
 template <int KIND>
 __global__ __launch_bounds__(256) void gemm_k64_kernel(GemmArgs g) {
     const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;

@@ -545,7 +545,10 @@ hipError_t launch(const MfmaScanArgs &a, hipStream_t st) {
 //            the gate); 48 channels 67 (73).  The least rounds x time wins: one
 //            block per CU of 16 channels up to 4096 channels, 32 up to 8192, 48
 //            up to 12288 and beyond (B64 x L512 x 4096 channels: 759 us, 855 with
-//            32-channel blocks).
+//            32-channel blocks).  Up to 256 steps and beyond one round, 32-channel
+//            blocks of 16-step chunks, two resident a CU: a block's start costs as
+//            much as its steps (B16 x L64 x 1536 16.9 -> 15.4 us, B32 x L256 x 4096
+//            205 -> 193, B64 x L128 x 4096 234 -> 204).
 //   N = 32   two states a lane; the model's 48-channel blocks beyond one round of
 //            16 (B8 x L200 x 1536 channels 32.8 against 34.9 us, B32 115 / 114)
 //   N = 64   four states a lane (two: B8 x L1000 x 1536 channels 200 against 174 us)
@@ -560,6 +563,7 @@ hipError_t launch_mfma_scan(int mode, int N, const MfmaScanArgs &a, hipStream_t 
     if (mode == kMScanModel) {
         if (N == 16) {
             if (33 * r16 <= 50 * r32 && 33 * r16 <= 67 * r48) return launch<kMScanModel, 16, 1, 1, 1, 64>(a, st);
+            if (r48 > 1 && a.L <= 256) return launch<kMScanModel, 16, 1, 1, 2, 16>(a, st);
             if (50 * r32 <= 67 * r48) return launch<kMScanModel, 16, 1, 1, 2, 32>(a, st);
             return launch<kMScanModel, 16, 1, 1, 3, 32>(a, st);
         }

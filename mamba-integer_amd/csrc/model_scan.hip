@@ -252,6 +252,7 @@ __global__ __launch_bounds__(kMThreads) void model_scan_kernel(MScanArgs a) {
     // stores, behind a third barrier.
     const int nchunks = (a.L + kMTC - 1) / kMTC;
     prefetch(0);
+    __syncthreads();   // s_dt is complete
     stash(0);
     if (nchunks > 1) prefetch(kMTC);
     __syncthreads();
@@ -371,6 +372,216 @@ struct SScanArgs {
     int B, L, D, H, P, s_y;
 };
 
+// Short sequences of many blocks (launch_ssd_scan): the lane layout of
+// model_scan_kernel (G lanes per channel, S = N/G states each, the update16
+// step); a block's CH channels lie in one head.  Per chunk the block stages x
+// and z (channel-major), the step decays (table lookup of the head's dt column)
+// and B, C: each 16-byte piece of a token's B (or C) row sums its squares, the
+// token's N/16 pieces (lanes of one quad) add up by DPP, and every piece is
+// scaled to the unit vector in Q7 before it lands in LDS.
+template <int N, int G>
+__global__ __launch_bounds__(kMThreads) void ssd_scan_kernel(SScanArgs a) {
+    constexpr int S = N / G;
+    constexpr int CH = kMThreads / G;
+    constexpr int XP = kMTC + 4;
+    constexpr int X16 = CH / 16;
+    constexpr int XPIECES = kMTC * X16;
+    constexpr int XPER = (XPIECES + kMThreads - 1) / kMThreads;
+    constexpr int BC16 = N / 16;
+    constexpr int BCPIECES = kMTC * BC16;
+    constexpr int BCPER = (BCPIECES + kMThreads - 1) / kMThreads;
+    static_assert(N % 16 == 0 && BC16 <= 4 && (S == 1 || S == 2 || S % 4 == 0), "state split");
+    static_assert(BCPIECES % 64 == 0 || BCPIECES < 64, "whole waves stage B and C");
+
+    __shared__ __align__(16) int8_t s_x[2][CH][XP];        // xs, z (channel-major)
+    __shared__ __align__(16) int32_t s_b[kMTC][N];
+    __shared__ __align__(16) int32_t s_c[kMTC][N];          // C * 2^16 (update16_cs)
+    __shared__ __align__(16) int2 s_y[kMTC][CH];
+    __shared__ __align__(16) int8_t s_o[kMTC][CH];
+    __shared__ __align__(16) int32_t s_n[kMTC];
+    __shared__ int32_t s_tab[256];
+    __shared__ int32_t s_gate[256];
+
+    const int tid = threadIdx.x;
+    const int ch = tid / G;
+    const int g = tid % G;
+    const int p0 = blockIdx.x * CH;
+    const int head = p0 / a.P;
+    const int b = blockIdx.y;
+    const int p = p0 + ch;
+
+    // doubled: the update takes n2 = 2n (table entries lie in [0, 2^15])
+    for (int i = tid; i < 255; i += kMThreads) s_tab[i] = 2 * a.tab[(int64_t)head * 255 + i];
+    for (int i = tid; i < 256; i += kMThreads) s_gate[i] = gate_q15(i - 128);
+
+    int32_t h[S];
+    {
+        const int64_t sidx = ((int64_t)b * a.D + p) * N + g * S;
+        for (int s = 0; s < S; ++s) h[s] = a.h_in ? a.h_in[sidx + s] : 0;
+    }
+
+    // ext_vector_type registers (a union-typed uint4 array touched through
+    // lambdas is kept in scratch)
+    v4i rx[2][XPER];
+    v4i rb[BCPER], rc[BCPER];
+    int dtv = 0;
+    const int64_t row0 = (int64_t)b * a.L;
+    const int64_t b_col = (int64_t)head * N, c_col = (int64_t)a.H * N + head * N, dt_col = 2 * (int64_t)a.H * N + head;
+    auto prefetch = [&](int t0) {
+        for (int j = 0; j < XPER; ++j) {
+            const int i = tid + j * kMThreads;
+            const int tt = i / X16, c16 = i % X16;
+            const bool ok = i < XPIECES && t0 + tt < a.L;
+            const int64_t rr = row0 + t0 + tt;
+            const v4i zero = v4i{0, 0, 0, 0};
+            rx[0][j] = ok ? *reinterpret_cast<const v4i *>(a.xs + rr * a.x_row + p0 + c16 * 16) : zero;
+            rx[1][j] = ok ? *reinterpret_cast<const v4i *>(a.z + rr * a.z_row + p0 + c16 * 16) : zero;
+        }
+        for (int j = 0; j < BCPER; ++j) {
+            const int i = tid + j * kMThreads;
+            const int tt = i / BC16, c16 = i % BC16;
+            const bool ok = i < BCPIECES && t0 + tt < a.L;
+            const int64_t off = (row0 + t0 + tt) * a.xp_row + c16 * 16;
+            rb[j] = ok ? *reinterpret_cast<const v4i *>(a.xp + off + b_col) : v4i{0, 0, 0, 0};
+            rc[j] = ok ? *reinterpret_cast<const v4i *>(a.xp + off + c_col) : v4i{0, 0, 0, 0};
+        }
+        dtv = (tid < kMTC && t0 + tid < a.L) ? a.xp[(row0 + t0 + tid) * a.xp_row + dt_col] : 0;
+    };
+    // sum of squares of a 16-byte piece of int8
+    auto sumsq = [](v4i v) {
+        const uint32_t w[4] = {(uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]};
+        int ss = 0;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int q = sb(w[e >> 2], e & 3);
+            ss += q * q;
+        }
+        return ss;
+    };
+    auto stash = [&]() {
+        for (int j = 0; j < XPER; ++j) {
+            const int i = tid + j * kMThreads;
+            if (i >= XPIECES) break;
+            const int tt = i / X16, c16 = i % X16;
+            const uint32_t wx[4] = {(uint32_t)rx[0][j][0], (uint32_t)rx[0][j][1], (uint32_t)rx[0][j][2],
+                                    (uint32_t)rx[0][j][3]};
+            const uint32_t wz[4] = {(uint32_t)rx[1][j][0], (uint32_t)rx[1][j][1], (uint32_t)rx[1][j][2],
+                                    (uint32_t)rx[1][j][3]};
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                s_x[0][c16 * 16 + e][tt] = (int8_t)sb(wx[e >> 2], e & 3);
+                s_x[1][c16 * 16 + e][tt] = (int8_t)sb(wz[e >> 2], e & 3);
+            }
+        }
+        for (int j = 0; j < BCPER; ++j) {
+            const int i = tid + j * kMThreads;
+            if (i - (tid & 63) >= BCPIECES) break;  // whole waves: the DPP sums below need every lane
+            const int tt = i / BC16, c16 = i % BC16;
+            // the token's pieces are BC16 adjacent lanes of one quad
+            int sbq = sumsq(rb[j]), scq = sumsq(rc[j]);
+            if constexpr (BC16 >= 2) {
+                sbq += __builtin_amdgcn_update_dpp(0, sbq, 0xB1, 0xF, 0xF, true);
+                scq += __builtin_amdgcn_update_dpp(0, scq, 0xB1, 0xF, 0xF, true);
+            }
+            if constexpr (BC16 >= 4) {
+                sbq += __builtin_amdgcn_update_dpp(0, sbq, 0x4E, 0xF, 0xF, true);
+                scq += __builtin_amdgcn_update_dpp(0, scq, 0x4E, 0xF, 0xF, true);
+            }
+            const int32_t ib = unit_inv(sbq), ic = unit_inv(scq);
+            const uint32_t wb[4] = {(uint32_t)rb[j][0], (uint32_t)rb[j][1], (uint32_t)rb[j][2], (uint32_t)rb[j][3]};
+            const uint32_t wc[4] = {(uint32_t)rc[j][0], (uint32_t)rc[j][1], (uint32_t)rc[j][2], (uint32_t)rc[j][3]};
+            if (i < BCPIECES) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    s_b[tt][c16 * 16 + e] = clamp32(rshr32(sb(wb[e >> 2], e & 3) * ib, 15), -127, 127);
+                    s_c[tt][c16 * 16 + e] = clamp32(rshr32(sb(wc[e >> 2], e & 3) * ic, 15), -127, 127) * 65536;
+                }
+            }
+        }
+        if (tid < kMTC) s_n[tid] = s_tab[clamp32(dtv, -127, 127) + 127];
+    };
+
+    // one step of this lane's S states: the exact int32 partials of y (the
+    // channel's G lanes are summed per group of four steps below)
+    auto step = [&](int t, int xv, int n2, int &yhi, int &ylo) {
+        int bv[S], cv[S];
+        if constexpr (S >= 4) {
+            for (int q = 0; q < S / 4; ++q) {
+                const int4 b4 = *reinterpret_cast<const int4 *>(&s_b[t][g * S + 4 * q]);
+                const int4 c4 = *reinterpret_cast<const int4 *>(&s_c[t][g * S + 4 * q]);
+                bv[4 * q] = b4.x; bv[4 * q + 1] = b4.y; bv[4 * q + 2] = b4.z; bv[4 * q + 3] = b4.w;
+                cv[4 * q] = c4.x; cv[4 * q + 1] = c4.y; cv[4 * q + 2] = c4.z; cv[4 * q + 3] = c4.w;
+            }
+        } else {
+            for (int s = 0; s < S; ++s) {
+                bv[s] = s_b[t][g * S + s];
+                cv[s] = s_c[t][g * S + s];
+            }
+        }
+        yhi = 0;
+        ylo = 0;
+        for (int s = 0; s < S; ++s) update16_cs(h[s], n2, bv[s], xv, cv[s], yhi, ylo);
+    };
+
+    const int32_t ylim = 100 << 18;
+    const int nchunks = (a.L + kMTC - 1) / kMTC;
+    prefetch(0);
+    for (int cidx = 0; cidx < nchunks; ++cidx) {
+        const int t0 = cidx * kMTC;
+        const int tn = min(kMTC, a.L - t0);
+        __syncthreads();
+        stash();
+        __syncthreads();
+        if (cidx + 1 < nchunks) prefetch(t0 + kMTC);
+        for (int t4 = 0; t4 < tn; t4 += 4) {
+            const uint32_t xw = *reinterpret_cast<const uint32_t *>(&s_x[0][ch][t4]);
+            const int4 n4 = *reinterpret_cast<const int4 *>(&s_n[t4]);
+            const int nv[4] = {n4.x, n4.y, n4.z, n4.w};
+            if (t4 + 4 <= tn) {
+                // the eight partials of the group reduced stage by stage across
+                // all eight: each DPP add reads a register written several
+                // instructions earlier, so it needs no wait states
+                int y[8];
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) step(t4 + tt, sb(xw, tt), nv[tt], y[2 * tt], y[2 * tt + 1]);
+                msum_all<G>(y);
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) s_y[t4 + tt][ch] = make_int2(y[2 * tt], y[2 * tt + 1]);
+            } else {
+                for (int tt = 0; tt < tn - t4; ++tt) {
+                    int y[2];
+                    step(t4 + tt, sb(xw, tt), s_n[t4 + tt], y[0], y[1]);
+                    msum_all<G>(y);
+                    s_y[t4 + tt][ch] = make_int2(y[0], y[1]);
+                }
+            }
+        }
+        __syncthreads();
+        for (int i = tid; i < kMTC * CH; i += kMThreads) {
+            const int tt = i / CH, cc = i % CH;
+            if (tt < tn) {
+                const int2 yv = s_y[tt][cc];
+                const int32_t y32 = clamp32(sat32_64(((int64_t)yv.x << 16) + yv.y), -ylim, ylim);
+                const int32_t gt = s_gate[s_x[1][cc][tt] + 128];
+                const int32_t yh = y32 >> 15, yl = y32 & 0x7fff;
+                const int32_t yg = yh * gt + (int32_t)(((uint32_t)yl * (uint32_t)gt) >> 15);
+                s_o[tt][cc] = (int8_t)clamp64(rshr64(yg, a.s_y), -127, 127);
+            }
+        }
+        __syncthreads();
+        for (int i = tid; i < kMTC * X16; i += kMThreads) {
+            const int tt = i / X16, c16 = i % X16;
+            if (tt < tn)
+                *reinterpret_cast<uint4 *>(a.yo + (row0 + t0 + tt) * a.x_row + p0 + c16 * 16) =
+                    *reinterpret_cast<const uint4 *>(&s_o[tt][c16 * 16]);
+        }
+    }
+    if (a.h_out) {
+        const int64_t sidx = ((int64_t)b * a.D + p) * N + g * S;
+        for (int s = 0; s < S; ++s) a.h_out[sidx + s] = h[s];
+    }
+}
+
 // One step of the SSD block scan (decode, len 1): block = 256/G channels of one
 // (sequence, head), G lanes per channel with S = N/G states each (the head's
 // P x N state is 16 KB at P = N = 64).  Wave 0 builds the token's unit-vector B and C (Q7)
@@ -480,6 +691,30 @@ hipError_t launch_ssd_scan(const int8_t *xs, const int8_t *xp, const int8_t *z, 
         }
         return hipGetLastError();
     }
+    // a block of the MFMA scan starts slower (tables, five waves' first loads and
+    // barriers): where three rounds or more of its 16-channel blocks would run 64
+    // steps or less, ssd_scan_kernel (24 heads of 64: B8 x L16 N64 15.9 against 10.6
+    // us, N32 10.2 / 8.8; B64 x L64 N64 167 / 135; past it B8 x L100 N64 34 / 38, B4 x
+    // L64 16.6 / 17.9); for N = 64 from one round on up to 32 steps (B4 x L16 11.4 /
+    // 8.7)
+    const int64_t blocks16 = (int64_t)B * (a.D / 16), cus = device_cus();
+    if ((L <= 64 && blocks16 >= 3 * cus) || (N == 64 && L <= 32 && blocks16 > cus)) {
+        int G = N / 4;
+        while (P % (kMThreads / G) != 0) G *= 2;  // P % 16 == 0, so G = 16 always fits
+        const dim3 grid((unsigned)(a.D / (kMThreads / G)), (unsigned)B);
+#define MI_SCASE(NN, GG)                                                                    \
+    if (N == NN && G == GG) {                                                               \
+        hipLaunchKernelGGL((ssd_scan_kernel<NN, GG>), grid, dim3(kMThreads), 0, st, a);     \
+        return hipGetLastError();                                                           \
+    }
+        MI_SCASE(16, 4)
+        MI_SCASE(16, 8)
+        MI_SCASE(16, 16)
+        MI_SCASE(32, 8)
+        MI_SCASE(32, 16)
+        MI_SCASE(64, 16)
+#undef MI_SCASE
+    }
     MfmaScanArgs m{};
     m.x = xs; m.z = z; m.b = xp; m.c = xp + (int64_t)H * N; m.dtc = xp + 2 * (int64_t)H * N; m.decay = tab; m.yo = yo;
     m.h_in = h_in; m.h_out = h_out;
@@ -492,9 +727,16 @@ hipError_t launch_model_scan(const int8_t *xs, const int8_t *dm, const int8_t *z
                              const int8_t *csrc, const int32_t *base, int8_t *yo, const int32_t *h_in, int32_t *h_out,
                              int64_t x_row, int64_t z_row, int64_t bc_row, int B, int L, int D, int N, int s_y,
                              hipStream_t st) {
-    // N = 64 (no model of this size): beyond two 16-channel blocks per CU, model_scan_kernel is faster (B8 x L1000 x 1536 channels 298 against
-    // 291 us, B32 x L200 212 against 257; B2 x L301 x 512 44 against 34)
-    if (N != 64 || (int64_t)B * ((D + 15) / 16) <= 2 * device_cus()) {
+    // model_scan_kernel: for N = 64 (no model of this size) beyond two 16-channel
+    // blocks per CU (B8 x L1000 x 1536 channels 298 against 291 us, B32 x L200 212
+    // against 257; B2 x L301 x 512 44 against 34); for N = 16 and 32 where 24
+    // rounds or more of such blocks would run 64 steps or less, since a block of the
+    // MFMA scan starts slower (N16, B64: L16 x 4096 channels 106 against 51 us, L64
+    // x 4096 154 / 108, L64 x 1536 60 / 47, L128 x 4096 204 / 212; N32, L16 x 4096
+    // 138 / 90, L64 x 1536 99 / 82)
+    const int64_t blocks16 = (int64_t)B * ((D + 15) / 16), cus = device_cus();
+    const bool many = blocks16 >= 24 * cus && L <= 64;
+    if (N == 64 ? blocks16 <= 2 * cus : !many) {
         MfmaScanArgs m{};
         m.x = xs; m.dm = dm; m.z = z; m.b = bsrc; m.c = csrc; m.decay = base; m.yo = yo; m.h_in = h_in; m.h_out = h_out;
         m.x_row = x_row; m.z_row = z_row; m.bc_row = bc_row; m.B = B; m.L = L; m.D = D; m.P = D; m.s_y = s_y;
@@ -504,9 +746,13 @@ hipError_t launch_model_scan(const int8_t *xs, const int8_t *dm, const int8_t *z
     a.xs = xs; a.dm = dm; a.z = z; a.bsrc = bsrc; a.csrc = csrc; a.base = base; a.yo = yo;
     a.h_in = h_in; a.h_out = h_out; a.x_row = x_row; a.z_row = z_row; a.bc_row = bc_row;
     a.B = B; a.L = L; a.D = D; a.s_y = s_y;
-    constexpr int CH = kMThreads / 16;
-    hipLaunchKernelGGL((model_scan_kernel<64, 16>), dim3((unsigned)((D + CH - 1) / CH), (unsigned)B), dim3(kMThreads), 0,
-                       st, a);
+    auto grid = [&](int ch) { return dim3((unsigned)((D + ch - 1) / ch), (unsigned)B); };
+    if (N == 16)
+        hipLaunchKernelGGL((model_scan_kernel<16, 4>), grid(kMThreads / 4), dim3(kMThreads), 0, st, a);
+    else if (N == 32)
+        hipLaunchKernelGGL((model_scan_kernel<32, 8>), grid(kMThreads / 8), dim3(kMThreads), 0, st, a);
+    else
+        hipLaunchKernelGGL((model_scan_kernel<64, 16>), grid(kMThreads / 16), dim3(kMThreads), 0, st, a);
     return hipGetLastError();
 }
 
