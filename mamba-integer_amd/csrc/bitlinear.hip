@@ -364,13 +364,16 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const ConvArgs &cv)
 
     GemmStage S;
     auto load = [&](int kt) {
-        const int off = kt * kBK + ac16 * 16 < g.K ? kt * kBK : 0;
+        // pieces past K read the start of their row (pa and pw lie in it: from
+        // there on a K below one stage would read past the row, past the last
+        // row's end too); their weights are zeroed
+        const int off = kt * kBK + ac16 * 16 < g.K ? kt * kBK : -16 * ac16;
         S.a0 = *reinterpret_cast<const v4i *>(pa[0] + off);
         S.a1 = *reinterpret_cast<const v4i *>(pa[1] + off);
         S.a2 = *reinterpret_cast<const v4i *>(pa[2] + off);
         S.a3 = *reinterpret_cast<const v4i *>(pa[3] + off);
         const bool wok = kt * (kBK / 16) + wh * 4 < g.kw;
-        S.w = *reinterpret_cast<const v4i *>(pw + (wok ? kt * (kBK / 16) : 0));
+        S.w = *reinterpret_cast<const v4i *>(pw + (wok ? kt * (kBK / 16) : -4 * wh));
         S.wmask = wok ? -1 : 0;
     };
     auto store_stage = [&](int buf) {
