@@ -27,8 +27,12 @@ struct MfmaScanArgs {
     int cs, nchunks_out;     // head mode
 };
 
+// A chunk's rows are addressed by 32-bit byte offsets, so rows stay below this:
+// 64 of them, as int32 outputs, below 2^31 bytes.
+constexpr int64_t kMfmaMaxRow = (int64_t)1 << 22;
+
 // N in {16, 32, 64} (channel and head modes also 128), decay shift 15, D and P
-// multiples of 16, 16-byte aligned rows, at least one step.
+// multiples of 16, 16-byte aligned rows shorter than kMfmaMaxRow, at least one step.
 hipError_t launch_mfma_scan(int mode, int N, const MfmaScanArgs &a, hipStream_t st);
 
 }  // namespace mi

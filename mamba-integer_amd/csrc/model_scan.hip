@@ -696,9 +696,10 @@ hipError_t launch_ssd_scan(const int8_t *xs, const int8_t *xp, const int8_t *z, 
     // steps or less, ssd_scan_kernel (24 heads of 64: B8 x L16 N64 15.9 against 10.6
     // us, N32 10.2 / 8.8; B64 x L64 N64 167 / 135; past it B8 x L100 N64 34 / 38, B4 x
     // L64 16.6 / 17.9); for N = 64 from one round on up to 32 steps (B4 x L16 11.4 /
-    // 8.7)
+    // 8.7).  Rows too long for the MFMA scan's offsets take it as well.
     const int64_t blocks16 = (int64_t)B * (a.D / 16), cus = device_cus();
-    if ((L <= 64 && blocks16 >= 3 * cus) || (N == 64 && L <= 32 && blocks16 > cus)) {
+    const bool wide = z_row >= kMfmaMaxRow || xp_row >= kMfmaMaxRow;   // (x_row <= z_row)
+    if (wide || (L <= 64 && blocks16 >= 3 * cus) || (N == 64 && L <= 32 && blocks16 > cus)) {
         int G = N / 4;
         while (P % (kMThreads / G) != 0) G *= 2;  // P % 16 == 0, so G = 16 always fits
         const dim3 grid((unsigned)(a.D / (kMThreads / G)), (unsigned)B);

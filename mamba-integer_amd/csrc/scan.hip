@@ -117,12 +117,11 @@ hipError_t launch_scan(const ScanArgs &a, int N, bool fast, hipStream_t st) {
     return hipGetLastError();
 }
 
-// row: the longest row stride of the call (a staged chunk of its rows, as int32
-// outputs, stays below 2^31 bytes)
+// row: the longest row stride of the call
 bool fast_shape(int N, int P, int k, int mode, int64_t row) {
     if (N != 16 && N != 32 && N != 64 && !(N == 128 && mode != kModeModel)) return false;
     if (P % 16 != 0) return false;
-    return k == 15 && row < (1 << 22);
+    return k == 15 && row < kMfmaMaxRow;
 }
 
 // ------------------------------------------------ float-compat reference
