@@ -74,23 +74,26 @@ class BitLinear(nn.Module):
             self.bias = nn.Parameter(torch.zeros(out_features))
         else:
             self.register_parameter("bias", None)
-        self._packed = {}        # k unit -> (packed weights, scale)
-        self._packed_key = None
+        self._packed = (None, {})
 
     # ------------------------------------------------------------ weights
     def _packed_weights(self, device, unit: int) -> Tuple[torch.Tensor, float]:
         """The packed ternary weights with k padded to a multiple of ``unit`` (16: the
         packing unit, the width of ``forward_int``'s rows; 64: four packed words,
-        which the kernels read at once), and their scale; kept per weight version."""
+        which the kernels read at once), and their scale; kept per weight version.
+        The key and its packings (by padded k) are replaced as one object, so a
+        call that packs for another key in between leaves this one's alone."""
         key = (self.weight._version, self.weight.data_ptr(), str(device))
-        if self._packed_key != key:
-            self._packed, self._packed_key = {}, key
-        if unit not in self._packed:
+        held = self._packed
+        if held[0] != key:
+            held = self._packed = (key, {})
+        kp = _ceil(self.in_features, unit)
+        if kp not in held[1]:
             w_quant, w_scale = weight_quant_ternary(self.weight.detach().to("cpu", torch.float32))
-            wq = torch.zeros((self.out_features, _ceil(self.in_features, unit)), dtype=torch.int8)
+            wq = torch.zeros((self.out_features, kp), dtype=torch.int8)
             wq[:, : self.in_features] = w_quant.to(torch.int8)
-            self._packed[unit] = ops.pack_ternary(wq.to(device)), float(w_scale)
-        return self._packed[unit]
+            held[1][kp] = ops.pack_ternary(wq.to(device)), float(w_scale)
+        return held[1][kp]
 
     @torch.no_grad()
     def get_ternary_weights(self) -> Tuple[torch.Tensor, torch.Tensor]:
