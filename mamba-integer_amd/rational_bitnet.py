@@ -111,9 +111,10 @@ class BitLinear(nn.Module):
         x2 = x.reshape(-1, self.in_features).to(torch.float32).contiguous()
         packed, w_scale = self._packed_weights(x.device, 64)
         bias = self.bias
-        # a float32 bias of the device is added by the GEMM's epilogue, any other
-        # by torch (with its promotion)
-        fused = bias is not None and bias.dtype == torch.float32 and bias.device == x.device and bias.is_contiguous()
+        # one float32 value a feature on the device is added by the GEMM's epilogue,
+        # any other bias by torch (with its promotion and broadcasting)
+        fused = (bias is not None and bias.shape == (self.out_features,) and bias.dtype == torch.float32
+                 and bias.device == x.device and bias.is_contiguous())
         y = ops.bitlinear_f32(x2, packed, w_scale, bias=bias if fused else None)
         if bias is not None and not fused:
             y = y + bias.to(y.device)
