@@ -30,7 +30,7 @@ import torch
 
 from mamba_int import ops
 
-_Q30 = torch.tensor(2.0 ** -30, dtype=torch.float32)
+_Q30 = torch.tensor(2.0 ** -30, dtype=torch.float32, device="cpu")   # (whatever the default device is at import)
 
 
 def _shift(shifts: Union[int, torch.Tensor]) -> int:
