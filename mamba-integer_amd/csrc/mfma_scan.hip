@@ -40,6 +40,8 @@
 //   SSD block     B2 x L1023, 24 x 64, N64    160 -> 73     B8 x L2048          592 -> 393
 //   head layout   B4 x L8192, 24 x 64, N128  2108 -> 1600
 //   channels      B1 x L256 x 512, N16         23 -> 10     B8 x L2048 x 1536   291 -> 116
+#include <stddef.h>
+
 #include <type_traits>
 
 #include "mfma_scan.hpp"
@@ -98,13 +100,17 @@ struct MfmaScan {
         int16_t b[2][N][TP];           // rows in the order of brow
         uint32_t c[2][TC][CP];         // C in all four bytes of a word
         int8_t dm[MODEL ? 2 : 1][MODEL ? CH : 1][TP];
-        int32_t n[SSD ? 2 : 1][SSD ? TC : 4];                 // decay of a step
-        int32_t y[2][NQ][2][TC][CH];   // hi and lo partials of a channel's scan waves
+        alignas(16) int32_t n[SSD ? 2 : 1][SSD ? TC : 4];     // decay of a step
+        alignas(16) int32_t y[2][NQ][2][TC][CH];   // hi and lo partials of a channel's scan waves
         int32_t csum[3][TC];           // 128 * sum of C over the states
         uint32_t dt[MODEL ? 256 : 1];  // by the raw byte of dm: dt << 16 | (clamped dm & 255)
         int32_t tab[SSD ? 255 : 1];
         int32_t gate[GATED ? 256 : 1]; // by the raw byte of z
     };
+    // read as 16-byte vectors
+    static_assert(offsetof(Smem, x) % 16 == 0 && offsetof(Smem, b) % 16 == 0 && offsetof(Smem, c) % 16 == 0 &&
+                  offsetof(Smem, n) % 16 == 0 && offsetof(Smem, y) % 16 == 0, "alignment");
+    static_assert(TP * 2 % 16 == 0 && CP * 4 % 16 == 0 && CH * 4 % 16 == 0, "row alignment");
 };
 
 template <int MODE, int N, int S, int M, int MW, int TC>
