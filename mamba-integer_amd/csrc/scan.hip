@@ -6,6 +6,8 @@
 // associative (the floor does not compose), so exact parallelism comes only
 // from independent lanes: (batch, head, channel, state).  Time stays
 // sequential inside every lane.
+#include <algorithm>
+
 #include "mi_common.hpp"
 #include "mfma_scan.hpp"
 
@@ -281,6 +283,54 @@ __global__ __launch_bounds__(64 * W) void elem_scan_kernel(const int32_t *u, con
     if (h_out && r == 0) h_out[b * C + c] = s;
 }
 
+// One lane per (sequence, channel), flat over both, the operands of A steps loaded
+// before the dependent chain runs over them (from clamped addresses; steps past the
+// end are skipped by a branch that is uniform): for sequences of few steps or
+// few channels, where elem_scan_kernel's rows and per-sequence blocks leave lanes
+// and loads idle (launch_elem_scan).
+template <bool CHUNKED, int A>
+__global__ __launch_bounds__(256) void elem_lane_kernel(const int32_t *u, const int32_t *n, int k, int cs, int32_t *h,
+                                                        int32_t *final_h, int32_t *dte, const int32_t *h_in,
+                                                        int32_t *h_out, int B, int L, int C, int nc) {
+    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= (int64_t)B * C) return;
+    const int64_t b = idx / C;
+    const int c = (int)(idx - b * C);
+    const int64_t base = b * L * C + c;
+    int32_t s = h_in ? h_in[idx] : 0;
+    int32_t p = 1 << 30;
+    int left = cs, chunk = 0;                     // steps left in the chunk
+    for (int t0 = 0; t0 < L; t0 += A) {
+        int32_t uu[A], nn[A];
+#pragma unroll
+        for (int j = 0; j < A; ++j) {
+            const int64_t off = base + (int64_t)min(t0 + j, L - 1) * C;
+            uu[j] = u[off];
+            nn[j] = n[off];
+        }
+#pragma unroll
+        for (int j = 0; j < A; ++j) {
+            const int t = t0 + j;
+            if (t < L) {
+                s = sat32_64((((int64_t)s * nn[j]) >> k) + (int64_t)uu[j]);
+                h[base + (int64_t)t * C] = s;
+                if constexpr (CHUNKED) {
+                    p = sat32_64(((int64_t)p * nn[j]) >> k);
+                    if (--left == 0 || t + 1 == L) {
+                        const int64_t co = (b * nc + chunk) * C + c;
+                        if (final_h) final_h[co] = s;
+                        if (dte) dte[co] = p;
+                        p = 1 << 30;
+                        left = cs;
+                        ++chunk;
+                    }
+                }
+            }
+        }
+    }
+    if (h_out) h_out[idx] = s;
+}
+
 template <bool CHUNKED, int R, int W>
 void launch_elem_rows(const int32_t *u, const int32_t *n, int k, int cs, int32_t *h, int32_t *final_h, int32_t *dte,
                       const int32_t *h_in, int32_t *h_out, int B, int L, int C, int nc, hipStream_t st) {
@@ -299,12 +349,35 @@ void launch_elem_scan(const int32_t *u, const int32_t *n, int k, int cs, int32_t
     // x 2048 104 / 142 / 192, 24576 x 2048 183 / 146 / 200, 65536 x 2048 432 / 319 /
     // 293.  A chunk ends with a group: fewer rows where four do not divide it.
     const int64_t lanes = (int64_t)B * C;
-    const int rows = lanes >= 49152 ? 1 : lanes >= 20480 ? 2 : 4;
     const int even = !CHUNKED || cs % 4 == 0 ? 4 : cs % 2 == 0 ? 2 : 1;
+    const int rows = std::min(lanes >= 49152 ? 1 : lanes >= 20480 ? 2 : 4, even);
+    // One lane per channel instead for few steps, where the rows' 16 groups ahead are
+    // mostly the last one again (rows / lanes, us: 32768 x 64 channels, 1 step 21.7 /
+    // 7.1, 16 steps 49.0 / 46.4; 512 x 32, 8 steps 3.1 / 2.7, 16 steps 3.4 / 3.4, 32
+    // steps 4.3 / 4.7), and for sequences that fill half a wave or less, up to a
+    // length that grows with the waves there are (rows / lanes: 2048 of them, 64 steps
+    // 0.9 to 1.04, 256 steps 0.5 to 0.8; 4096, 256 steps 0.85 with four rows, 1.1 to 1.4
+    // with one or two; 8192, 1000 steps 1.14 to 1.9).  Four steps and fewer: one load
+    // ahead (eight repeat the last).  Blocks of 64 lanes where there are few, and in
+    // the chunked form (32768 x 3, 64 steps 27 us, 33 with 256 lanes; elementwise 8192
+    // x 100, 16 steps 26 with 64, 21 with 256).
+    const int64_t cw = 64 / rows, waves = std::min<int64_t>(B * ((C + cw - 1) / cw), 1 << 20);
+    if (L < (rows == 4 ? 16 : 32) || (2 * (int64_t)C <= cw && (waves * waves * waves) >> (rows == 4 ? 29 : 27) >= L)) {
+        const bool one = L < 4 || (!CHUNKED && L == 4);
+        const unsigned threads = one || (!CHUNKED && lanes >= 65536) ? 256 : 64;
+        const dim3 grid((unsigned)((lanes + threads - 1) / threads));
+        if (one)
+            hipLaunchKernelGGL((elem_lane_kernel<CHUNKED, 1>), grid, dim3(threads), 0, st, u, n, k, cs, h, final_h, dte,
+                               h_in, h_out, B, L, C, nc);
+        else
+            hipLaunchKernelGGL((elem_lane_kernel<CHUNKED, 8>), grid, dim3(threads), 0, st, u, n, k, cs, h, final_h, dte,
+                               h_in, h_out, B, L, C, nc);
+        return;
+    }
     auto go = [&](auto f) { f(u, n, k, cs, h, final_h, dte, h_in, h_out, B, L, C, nc, st); };
-    if (rows == 4 && even == 4)
+    if (rows == 4)
         go(lanes > 8192 ? launch_elem_rows<CHUNKED, 4, 4> : launch_elem_rows<CHUNKED, 4, 2>);
-    else if (rows >= 2 && even >= 2)
+    else if (rows == 2)
         go(launch_elem_rows<CHUNKED, 2, 4>);
     else
         go(launch_elem_rows<CHUNKED, 1, 4>);
