@@ -2,6 +2,9 @@
 // matrix cores (mfma_scan.hip).
 #pragma once
 
+#include <initializer_list>
+#include <utility>
+
 #include "mi_common.hpp"
 
 namespace mi {
@@ -26,6 +29,15 @@ struct MfmaScanArgs {
     int s_y;                 // gated modes
     int cs, nchunks_out;     // head mode
 };
+
+// The steps of the first row of a table (rounds up to, steps) that r lies in, 0 past
+// the last: how long sequences a VALU kernel takes instead of the MFMA scan.
+constexpr double kAnyRounds = 1e30;
+inline int steps_at(std::initializer_list<std::pair<double, int>> table, double r) {
+    for (const auto &e : table)
+        if (r <= e.first) return e.second;
+    return 0;
+}
 
 // A chunk's rows are addressed by 32-bit byte offsets, so rows stay below this:
 // 64 of them, as int32 outputs, below 2^31 bytes.

@@ -2,8 +2,9 @@
 // decay from base + dm, dt from dm, input xs*dt (x) B, the exact floor
 // recurrence, y = C.h, the gate by z and the requant of the out_proj input.
 //
-// (mfma_scan.hip has the form that most shapes take; this one remains for N = 64
-// at many channels.)
+// (mfma_scan.hip has the form that most shapes take; this one remains for short
+// sequences, where launch_model_scan measured it faster, and for N = 64 at many
+// channels.)
 //
 // Layout: a block of 256 threads owns CH = 256/G channels of one sequence; G
 // adjacent lanes share a channel and keep S = N/G states each in VGPRs (read
@@ -361,7 +362,8 @@ __global__ __launch_bounds__(kMThreads) void model_scan_kernel(MScanArgs a) {
 
 // ------------------------------------------------ SSD block scan (V2)
 // The scan of MambaIntegerBlockV2 (spec rules 7.4-7.8; ssd_multihead.py:
-// 536-586) is mfma_scan.hip's; one decode step (len 1) has its own kernel here.
+// 536-586): mfma_scan.hip has the form for longer sequences, ssd_scan_kernel the one
+// for short ones (launch_ssd_scan), and one decode step (len 1) a kernel of its own.
 struct SScanArgs {
     const int8_t *xs, *z, *xp;     // [B*L rows][row stride]; z points at its first column
     const int32_t *tab;            // [H][255]
@@ -372,7 +374,7 @@ struct SScanArgs {
     int B, L, D, H, P, s_y;
 };
 
-// Short sequences of many blocks (launch_ssd_scan): the lane layout of
+// Short sequences and very long rows: the lane layout of
 // model_scan_kernel (G lanes per channel, S = N/G states each, the update16
 // step); a block's CH channels lie in one head.  Per chunk the block stages x
 // and z (channel-major), the step decays (table lookup of the head's dt column)
@@ -692,14 +694,17 @@ hipError_t launch_ssd_scan(const int8_t *xs, const int8_t *xp, const int8_t *z, 
         return hipGetLastError();
     }
     // a block of the MFMA scan starts slower (tables, five waves' first loads and
-    // barriers): where three rounds or more of its 16-channel blocks would run 64
-    // steps or less, ssd_scan_kernel (24 heads of 64: B8 x L16 N64 15.9 against 10.6
-    // us, N32 10.2 / 8.8; B64 x L64 N64 167 / 135; past it B8 x L100 N64 34 / 38, B4 x
-    // L64 16.6 / 17.9); for N = 64 from one round on up to 32 steps (B4 x L16 11.4 /
-    // 8.7).  Rows too long for the MFMA scan's offsets take it as well.
-    const int64_t blocks16 = (int64_t)B * (a.D / 16), cus = device_cus();
+    // barriers): ssd_scan_kernel up to these steps, by rounds of 16-channel blocks
+    // over CUs (MFMA / this, heads of 64: N16 3 rounds, 8 steps 1.10, 32 steps 0.74, 12
+    // rounds, 48 steps 1.21; N32 3 rounds, 16 steps 1.20, 32 steps 0.89; N64 one round,
+    // 16 steps 1.01, 32 steps 0.81, two rounds, 48 steps 1.04, 64 steps 0.89, 12
+    // rounds, 100 steps 1.03), and for rows too long for the MFMA scan's offsets
+    const double r = (double)B * (a.D / 16) / device_cus();
+    const int steps = N == 16   ? steps_at({{1.9, 4}, {3.9, 12}, {8, 24}, {kAnyRounds, 56}}, r)
+                      : N == 32 ? steps_at({{1, 2}, {2, 8}, {3.9, 16}, {5, 24}, {kAnyRounds, 48}}, r)
+                                : steps_at({{1, 16}, {3.9, 48}, {5, 64}, {9, 80}, {kAnyRounds, 100}}, r);
     const bool wide = z_row >= kMfmaMaxRow || xp_row >= kMfmaMaxRow;   // (x_row <= z_row)
-    if (wide || (L <= 64 && blocks16 >= 3 * cus) || (N == 64 && L <= 32 && blocks16 > cus)) {
+    if (wide || L <= steps) {
         int G = N / 4;
         while (P % (kMThreads / G) != 0) G *= 2;  // P % 16 == 0, so G = 16 always fits
         const dim3 grid((unsigned)(a.D / (kMThreads / G)), (unsigned)B);
@@ -728,16 +733,21 @@ hipError_t launch_model_scan(const int8_t *xs, const int8_t *dm, const int8_t *z
                              const int8_t *csrc, const int32_t *base, int8_t *yo, const int32_t *h_in, int32_t *h_out,
                              int64_t x_row, int64_t z_row, int64_t bc_row, int B, int L, int D, int N, int s_y,
                              hipStream_t st) {
-    // model_scan_kernel: for N = 64 (no model of this size) beyond two 16-channel
-    // blocks per CU (B8 x L1000 x 1536 channels 298 against 291 us, B32 x L200 212
-    // against 257; B2 x L301 x 512 44 against 34); for N = 16 and 32 where 24
-    // rounds or more of such blocks would run 64 steps or less, since a block of the
-    // MFMA scan starts slower (N16, B64: L16 x 4096 channels 106 against 51 us, L64
-    // x 4096 154 / 108, L64 x 1536 60 / 47, L128 x 4096 204 / 212; N32, L16 x 4096
-    // 138 / 90, L64 x 1536 99 / 82)
-    const int64_t blocks16 = (int64_t)B * ((D + 15) / 16), cus = device_cus();
-    const bool many = blocks16 >= 24 * cus && L <= 64;
-    if (N == 64 ? blocks16 <= 2 * cus : !many) {
+    // model_scan_kernel where a block of the MFMA scan starts slower than its steps
+    // win back, by rounds of 16-channel blocks over CUs (MFMA / this: N16 1 round, 4
+    // steps 1.02, 8 steps 0.99, 3 rounds, 16 steps 1.05, 8 and 16 rounds, 64 steps 1.07
+    // and 1.09, 100 steps 0.99; N32 1.5 rounds, 100 steps 1.03, 3 rounds, 16 steps 1.02,
+    // 32 steps 0.87, 6 rounds, 64 steps 1.06, 16 rounds, 100 steps 1.11; N64 1 round, 16
+    // steps 1.04, 32 steps 0.94, 2 rounds, 100 steps 1.06), at any length where its
+    // 48-channel blocks make two rounds of 16 channels' four (N32: 1.13 at 400 steps)
+    // and for N = 64 (no model of this size) beyond two rounds (16 rounds, 400 steps
+    // 1.08); and for rows too long for the MFMA scan's offsets
+    const double r = (double)B * ((D + 15) / 16) / device_cus();
+    const int steps = N == 16   ? steps_at({{1, 4}, {2, 12}, {3, 16}, {4.2, 8}, {7, 16}, {9, 64}, {11, 16}, {40, 64}, {kAnyRounds, 112}}, r)
+                      : N == 32 ? steps_at({{1, 4}, {2, 112}, {3, 16}, {4, INT32_MAX}, {7, 64}, {kAnyRounds, 112}}, r)
+                                : steps_at({{1, 24}, {2, 112}, {kAnyRounds, INT32_MAX}}, r);
+    const bool wide = z_row >= kMfmaMaxRow || bc_row >= kMfmaMaxRow;   // (x_row <= z_row)
+    if (!wide && L > steps) {
         MfmaScanArgs m{};
         m.x = xs; m.dm = dm; m.z = z; m.b = bsrc; m.c = csrc; m.decay = base; m.yo = yo; m.h_in = h_in; m.h_out = h_out;
         m.x_row = x_row; m.z_row = z_row; m.bc_row = bc_row; m.B = B; m.L = L; m.D = D; m.P = D; m.s_y = s_y;
@@ -748,7 +758,11 @@ hipError_t launch_model_scan(const int8_t *xs, const int8_t *dm, const int8_t *z
     a.h_in = h_in; a.h_out = h_out; a.x_row = x_row; a.z_row = z_row; a.bc_row = bc_row;
     a.B = B; a.L = L; a.D = D; a.s_y = s_y;
     auto grid = [&](int ch) { return dim3((unsigned)((D + ch - 1) / ch), (unsigned)B); };
-    if (N == 16)
+    // (two states a lane while its blocks of 32 channels fill the CUs no more than
+    // twice: 2 rounds, 8 steps 4.6 us, 5.3 with four)
+    if (N == 16 && r <= 4.2)
+        hipLaunchKernelGGL((model_scan_kernel<16, 8>), grid(kMThreads / 8), dim3(kMThreads), 0, st, a);
+    else if (N == 16)
         hipLaunchKernelGGL((model_scan_kernel<16, 4>), grid(kMThreads / 4), dim3(kMThreads), 0, st, a);
     else if (N == 32)
         hipLaunchKernelGGL((model_scan_kernel<32, 8>), grid(kMThreads / 8), dim3(kMThreads), 0, st, a);

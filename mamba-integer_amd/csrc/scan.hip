@@ -7,6 +7,7 @@
 // from independent lanes: (batch, head, channel, state).  Time stays
 // sequential inside every lane.
 #include <algorithm>
+#include <type_traits>
 
 #include "mi_common.hpp"
 #include "mfma_scan.hpp"
@@ -14,7 +15,8 @@
 namespace mi {
 namespace {
 
-// chunk lengths of chunk_states that the fast kernels take (their staged chunks divide it)
+// steps that scan_kernel stages at a time; chunk lengths of chunk_states are multiples
+// of it in the fast kernels (their staged chunks divide it)
 constexpr int kTC = 64;
 
 enum ScanMode { kModeChannel = 0, kModeHead = 1, kModeModel = 2 };
@@ -101,29 +103,361 @@ __global__ __launch_bounds__(256) void scan_generic_kernel(ScanArgs a, int N) {
         for (int n = 0; n < N; ++n) a.h_out[sidx + n] = h[n];
 }
 
-// ------------------------------------------------------------- dispatch
-template <int MODE>
-hipError_t launch_scan(const ScanArgs &a, int N, bool fast, hipStream_t st) {
-    // (the model mode's fast shapes go through launch_model_scan; here it takes
-    // the generic kernel only)
-    if constexpr (MODE != kModeModel) {
-        if (fast) {
-            MfmaScanArgs m{};
-            m.x = a.x; m.b = a.bsrc; m.c = a.csrc; m.decay = a.decay; m.y = a.y; m.chunk_states = a.chunk_states; m.h_in = a.h_in; m.h_out = a.h_out;
-            m.x_row = a.x_row; m.bc_row = a.bc_row; m.B = a.B; m.L = a.L; m.D = a.H * a.P; m.P = a.P; m.cs = a.cs; m.nchunks_out = a.nchunks_out;
-            return launch_mfma_scan(MODE == kModeChannel ? kMScanChannel : kMScanHead, N, m, st);
+// -------------------------------------------------- VALU scan, short calls
+// The channel and head layouts where a sequence has few steps (launch_scan has the
+// lengths: a block of the MFMA scan starts slower, with its helper waves' staging, a
+// barrier a chunk and mostly one block a CU) or rows too long for that kernel's
+// offsets.  A block owns CH = 256/G channels of one (batch,
+// head); G adjacent lanes share a channel and hold S = N/G states each, read as two
+// 16-bit fields by the update (update16); their partial y sums are combined by DPP.
+// Inputs of 64 steps go through LDS, x transposed to channel-major so one
+// ds_read_b32 serves four steps, outputs leave through LDS in 16-byte stores.
+constexpr int kThreads = 256;
+
+// Sums of K independent values over the G adjacent lanes of a channel, stage by
+// stage across all K (a DPP add then reads a register written K instructions
+// earlier, so no wait states); every lane gets them.
+template <int G, int K>
+__device__ __forceinline__ void group_sums(int (&v)[K]) {
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        if constexpr (G >= 2) v[k] += __builtin_amdgcn_update_dpp(0, v[k], 0xB1, 0xF, 0xF, false);   // quad_perm 1,0,3,2
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        if constexpr (G >= 4) v[k] += __builtin_amdgcn_update_dpp(0, v[k], 0x4E, 0xF, 0xF, false);   // quad_perm 2,3,0,1
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        if constexpr (G >= 8) v[k] += __builtin_amdgcn_update_dpp(0, v[k], 0x141, 0xF, 0xF, false);  // row_half_mirror
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        if constexpr (G >= 16) v[k] += __builtin_amdgcn_update_dpp(0, v[k], 0x140, 0xF, 0xF, false); // row_mirror
+}
+
+__device__ __forceinline__ int sbyte(uint32_t w, int i) { return (int)(int8_t)(w >> (8 * i)); }
+
+// Loads 16 consecutive bytes (16-byte aligned) or zeros when out of range.
+__device__ __forceinline__ uint4 load16(const int8_t *p, bool ok) {
+    if (ok) return *reinterpret_cast<const uint4 *>(p);
+    return make_uint4(0, 0, 0, 0);
+}
+
+template <int N, int G, int MODE>
+__global__ __launch_bounds__(kThreads) void scan_kernel(ScanArgs a) {
+    static_assert(MODE != kModeModel, "the fused model scan has its own kernel (model_scan.hip)");
+    constexpr int S = N / G;
+    constexpr int CH = kThreads / G;
+    constexpr int XP = kTC + 4;                 // padded row of the transposed x tile
+    constexpr int X16 = CH / 16;                // 16-byte pieces per time row of x
+    constexpr int XPIECES = kTC * X16;          // per chunk
+    constexpr int XPER = (XPIECES + kThreads - 1) / kThreads;
+    constexpr int BC16 = N / 16;
+    constexpr int BCPIECES = kTC * BC16;
+    constexpr int BCPER = (BCPIECES + kThreads - 1) / kThreads;
+
+    __shared__ __align__(16) int8_t s_x[CH][XP];
+    // WIDEB: B widened to int32, so the input term B * x and the saturating
+    // add are one clamped v_mad_i32_i24 (which takes no SDWA byte select).
+    // Lanes of one or two states keep B as bytes: their latency-bound chain
+    // measured slower with the wider staging (config 1: 22.0 -> 25.1 us)
+    constexpr bool WIDEB = S >= 4;
+    constexpr bool STAGE_Y = CH <= 64;  // int32 y staged in LDS (16 KB at most)
+    // blocks of <= 32 channels (G >= 8) reduce the y partials of four steps
+    // together and park the exact (yhi, ylo) pairs here; the chunk epilogue
+    // recombines and saturates once per (step, channel)
+    constexpr bool DEFER = CH <= 32;
+    // C32: C staged as int32 C * 2^16 as well (update16_cs: y's high partial in one
+    // v_dot2c, no byte extraction per state), in the channel layout (64 rounds of N =
+    // 16, 48 steps 73 -> 66 us) where two blocks a CU still fit
+    constexpr int kLdsC32 = CH * (kTC + 4) + 2 * kTC * N * 4 + (STAGE_Y ? kTC * CH * 4 : 16) + (DEFER ? kTC * CH * 8 : 8);
+    constexpr bool C32 = WIDEB && MODE == kModeChannel && kLdsC32 <= 81920;
+    __shared__ __align__(16) std::conditional_t<WIDEB, int32_t, int8_t> s_b[kTC][N];
+    __shared__ __align__(16) std::conditional_t<C32, int32_t, int8_t> s_c[kTC][N];
+    __shared__ __align__(16) int32_t s_o32[STAGE_Y ? kTC : 1][STAGE_Y ? CH : 4];
+    __shared__ __align__(16) int2 s_y[DEFER ? kTC : 1][DEFER ? CH : 1];
+
+    const int tid = threadIdx.x;
+    const int ch = tid / G;
+    const int g = tid % G;
+    const int p0 = blockIdx.x * CH;
+    const int hd = blockIdx.y;
+    const int b = blockIdx.z;
+    const int p = p0 + ch;
+    const bool active = p < a.P;
+
+    // ---- per-thread constants and state
+    int32_t n2[S];  // 2n: the update16 form takes the doubled decay
+    int32_t h[S];
+    {
+        const int64_t sidx = ((((int64_t)b * a.H + hd) * a.P + (active ? p : 0)) * N) + g * S;
+        for (int s = 0; s < S; ++s) {
+            h[s] = (a.h_in && active) ? a.h_in[sidx + s] : 0;
+            if constexpr (MODE == kModeChannel)
+                n2[s] = 2 * (active ? a.decay[(int64_t)p * N + g * S + s] : 0);
+            else
+                n2[s] = 2 * a.decay[hd];
         }
     }
+
+    // ---- staging registers
+    uint4 rx[XPER];
+    uint4 rb[BCPER], rc[BCPER];
+    const int64_t row0 = (int64_t)b * a.L;  // first (b, t=0) row index
+
+    auto prefetch = [&](int t0) {
+        for (int j = 0; j < XPER; ++j) {
+            const int i = tid + j * kThreads;
+            const int tt = i / X16, c16 = i % X16;
+            const bool ok = i < XPIECES && t0 + tt < a.L && p0 + c16 * 16 < a.P;
+            rx[j] = load16(a.x + (row0 + t0 + tt) * a.x_row + (int64_t)hd * a.P + p0 + c16 * 16, ok);
+        }
+        for (int j = 0; j < BCPER; ++j) {
+            const int i = tid + j * kThreads;
+            const int tt = i / BC16, c16 = i % BC16;
+            const bool ok = i < BCPIECES && t0 + tt < a.L;
+            const int64_t off = (row0 + t0 + tt) * a.bc_row + (MODE == kModeHead ? (int64_t)hd * N : 0) + c16 * 16;
+            rb[j] = load16(a.bsrc + off, ok);
+            rc[j] = load16(a.csrc + off, ok);
+        }
+    };
+    auto stash = [&]() {
+        for (int j = 0; j < XPER; ++j) {
+            const int i = tid + j * kThreads;
+            if (i >= XPIECES) break;
+            const int tt = i / X16, c16 = i % X16;
+            const uint32_t w[4] = {rx[j].x, rx[j].y, rx[j].z, rx[j].w};
+            for (int e = 0; e < 16; ++e) s_x[c16 * 16 + e][tt] = (int8_t)(w[e >> 2] >> (8 * (e & 3)));
+        }
+        for (int j = 0; j < BCPER; ++j) {
+            const int i = tid + j * kThreads;
+            if (i >= BCPIECES) break;
+            const int tt = i / BC16, c16 = i % BC16;
+            if constexpr (WIDEB) {
+                const uint32_t w[4] = {rb[j].x, rb[j].y, rb[j].z, rb[j].w};
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<int4 *>(&s_b[tt][c16 * 16 + 4 * q]) =
+                        make_int4(sbyte(w[q], 0), sbyte(w[q], 1), sbyte(w[q], 2), sbyte(w[q], 3));
+            } else {
+                *reinterpret_cast<uint4 *>(&s_b[tt][c16 * 16]) = rb[j];
+            }
+            if constexpr (C32) {
+                const uint32_t w[4] = {rc[j].x, rc[j].y, rc[j].z, rc[j].w};
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<int4 *>(&s_c[tt][c16 * 16 + 4 * q]) = make_int4(
+                        sbyte(w[q], 0) * 65536, sbyte(w[q], 1) * 65536, sbyte(w[q], 2) * 65536, sbyte(w[q], 3) * 65536);
+            } else {
+                *reinterpret_cast<uint4 *>(&s_c[tt][c16 * 16]) = rc[j];
+            }
+        }
+    };
+
+    // one step of this lane's S states: the exact int32 partials of y
+    auto step = [&](int t, int xv, int &yhi, int &ylo) {
+        yhi = 0;
+        ylo = 0;
+        if constexpr (C32) {
+            // every coefficient read first, then the S updates
+            int bv[S], cv[S];
+#pragma unroll
+            for (int q = 0; q < S / 4; ++q) {
+                const int4 b4 = *reinterpret_cast<const int4 *>(&s_b[t][g * S + 4 * q]);
+                const int4 c4 = *reinterpret_cast<const int4 *>(&s_c[t][g * S + 4 * q]);
+                bv[4 * q] = b4.x; bv[4 * q + 1] = b4.y; bv[4 * q + 2] = b4.z; bv[4 * q + 3] = b4.w;
+                cv[4 * q] = c4.x; cv[4 * q + 1] = c4.y; cv[4 * q + 2] = c4.z; cv[4 * q + 3] = c4.w;
+            }
+#pragma unroll
+            for (int s = 0; s < S; ++s) update16_cs(h[s], n2[s], bv[s], xv, cv[s], yhi, ylo);
+        } else if constexpr (WIDEB) {
+            // every coefficient read first, then the S updates
+            int bv[S];
+            uint32_t cw[S / 4];
+#pragma unroll
+            for (int q = 0; q < S / 4; ++q) {
+                const int4 b4 = *reinterpret_cast<const int4 *>(&s_b[t][g * S + 4 * q]);
+                bv[4 * q] = b4.x; bv[4 * q + 1] = b4.y; bv[4 * q + 2] = b4.z; bv[4 * q + 3] = b4.w;
+                cw[q] = *reinterpret_cast<const uint32_t *>(&s_c[t][g * S + 4 * q]);
+            }
+#pragma unroll
+            for (int s = 0; s < S; ++s) update16_b(h[s], n2[s], bv[s], xv, sbyte(cw[s >> 2], s & 3), yhi, ylo);
+        } else {
+            uint32_t bw = 0, cw = 0;
+            for (int s = 0; s < S; ++s) {
+                bw |= (uint32_t)(uint8_t)s_b[t][g * S + s] << (8 * s);
+                cw |= (uint32_t)(uint8_t)s_c[t][g * S + s] << (8 * s);
+            }
+#pragma unroll
+            for (int s = 0; s < S; ++s) update16(h[s], n2[s], __mul24(sbyte(bw, s), xv), sbyte(cw, s), yhi, ylo);
+        }
+    };
+
+    const int nchunks = (a.L + kTC - 1) / kTC;
+    prefetch(0);
+    for (int cidx = 0; cidx < nchunks; ++cidx) {
+        const int t0 = cidx * kTC;
+        const int tn = min(kTC, a.L - t0);
+        __syncthreads();
+        stash();
+        __syncthreads();
+        if (cidx + 1 < nchunks) prefetch(t0 + kTC);
+
+        for (int t4 = 0; t4 < tn; t4 += 4) {
+            const uint32_t xw = *reinterpret_cast<const uint32_t *>(&s_x[ch][t4]);
+            const int tend = min(4, tn - t4);
+            if constexpr (DEFER) {
+                if (tend == 4) {
+                    int y[8];
+#pragma unroll
+                    for (int tt = 0; tt < 4; ++tt) step(t4 + tt, sbyte(xw, tt), y[2 * tt], y[2 * tt + 1]);
+                    group_sums<G>(y);
+#pragma unroll
+                    for (int tt = 0; tt < 4; ++tt) s_y[t4 + tt][ch] = make_int2(y[2 * tt], y[2 * tt + 1]);
+                } else {
+                    for (int tt = 0; tt < tend; ++tt) {
+                        int y[2];
+                        step(t4 + tt, sbyte(xw, tt), y[0], y[1]);
+                        group_sums<G>(y);
+                        s_y[t4 + tt][ch] = make_int2(y[0], y[1]);
+                    }
+                }
+                continue;
+            }
+            for (int tt = 0; tt < tend; ++tt) {
+                const int t = t4 + tt;
+                int y[2];
+                step(t, sbyte(xw, tt), y[0], y[1]);
+                group_sums<G>(y);
+                const int32_t y32 = sat32_64(((int64_t)y[0] << 16) + y[1]);
+                if (g == 0) {
+                    if constexpr (STAGE_Y) s_o32[t][ch] = y32;
+                    else if (active) a.y[(row0 + t0 + t) * a.x_row + (int64_t)hd * a.P + p] = y32;
+                }
+            }
+        }
+        __syncthreads();
+        if constexpr (DEFER) {
+            // chunk epilogue: y = sat32(yhi * 2^16 + ylo)
+            for (int i = tid; i < kTC * CH; i += kThreads) {
+                const int tt = i / CH, cc = i % CH;
+                if (tt < tn) {
+                    const int2 yv = s_y[tt][cc];
+                    s_o32[tt][cc] = sat32_64(((int64_t)yv.x << 16) + yv.y);
+                }
+            }
+            __syncthreads();
+        }
+        // ---- write the staged outputs of this chunk
+        if constexpr (STAGE_Y) {
+            constexpr int Y4 = CH / 4;
+            for (int i = tid; i < kTC * Y4; i += kThreads) {
+                const int tt = i / Y4, c4 = i % Y4;
+                if (tt < tn && p0 + c4 * 4 < a.P)
+                    *reinterpret_cast<uint4 *>(a.y + (row0 + t0 + tt) * a.x_row + (int64_t)hd * a.P + p0 + c4 * 4) =
+                        *reinterpret_cast<const uint4 *>(&s_o32[tt][c4 * 4]);
+            }
+        }
+        if constexpr (MODE == kModeHead) {
+            // chunk_states at every multiple of cs (cs is a multiple of kTC) and at the end
+            const int tdone = t0 + tn;
+            if (a.chunk_states && active && (tdone % a.cs == 0 || tdone == a.L)) {
+                const int cc = (tdone - 1) / a.cs;
+                int32_t *dst = a.chunk_states +
+                               ((((int64_t)b * a.nchunks_out + cc) * a.H + hd) * a.P + p) * N + g * S;
+                for (int s = 0; s < S; ++s) dst[s] = h[s];
+            }
+        }
+    }
+    if (a.h_out && active) {
+        const int64_t sidx = ((((int64_t)b * a.H + hd) * a.P + p) * N) + g * S;
+        for (int s = 0; s < S; ++s) a.h_out[sidx + s] = h[s];
+    }
+}
+
+
+// Lanes per channel: enough waves to cover the 1024 SIMDs when possible.
+int pick_g(int N, int64_t channels) {
+    int g = 1;
+    while (g < 16 && N % (2 * g) == 0 && (N / g > 32 || channels * g / 64 < 1024)) g *= 2;
+    return g;
+}
+
+template <int N, int MODE>
+hipError_t launch_valu_n(const ScanArgs &a, hipStream_t st) {
+    auto grid = [&](int ch) { return dim3((unsigned)((a.P + ch - 1) / ch), (unsigned)a.H, (unsigned)a.B); };
+    const int g = pick_g(N, (int64_t)a.B * a.H * a.P);
+#define MI_CASE_G(GG)                                                                                     \
+    if constexpr (N / GG <= 32)                                                                           \
+        if (g == GG) hipLaunchKernelGGL((scan_kernel<N, GG, MODE>), grid(kThreads / GG), dim3(kThreads), 0, st, a);
+    MI_CASE_G(1)
+    MI_CASE_G(2)
+    MI_CASE_G(4)
+    MI_CASE_G(8)
+    MI_CASE_G(16)
+#undef MI_CASE_G
+    return hipGetLastError();
+}
+
+template <int MODE>
+hipError_t launch_valu_scan(const ScanArgs &a, int N, hipStream_t st) {
+    switch (N) {
+        case 16: return launch_valu_n<16, MODE>(a, st);
+        case 32: return launch_valu_n<32, MODE>(a, st);
+        case 64: return launch_valu_n<64, MODE>(a, st);
+        default: return launch_valu_n<128, MODE>(a, st);
+    }
+}
+
+// ------------------------------------------------------------- dispatch
+template <int MODE>
+hipError_t launch_generic(const ScanArgs &a, int N, hipStream_t st) {
     const int64_t lanes = (int64_t)a.B * a.H * a.P;
     hipLaunchKernelGGL((scan_generic_kernel<MODE>), dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, st, a, N);
     return hipGetLastError();
 }
 
-// row: the longest row stride of the call
-bool fast_shape(int N, int P, int k, int mode, int64_t row) {
+// Longest sequences that scan_kernel takes, by rounds: 16-channel blocks over CUs.
+// Measured with both kernels over 1 to 128 steps (MFMA / VALU, us a call):
+//   channels  N16   1 round, 1 step 3.6 / 3.0, 8 steps 3.7 / 3.4, 16 steps 4.0 / 3.9,
+//                   32 steps 4.7 / 5.1; 64 rounds, 16 steps 54 / 39, 48 steps 76 / 66
+//             N32   1 round, 8 steps 4.0 / 3.6, 16 steps 4.4 / 4.3
+//             N64   1 round, 8 steps 4.7 / 4.3, 16 steps 5.3 / 5.2; 2 rounds never
+//             N128  3 rounds only (32-channel blocks make one and a half): 8 steps, 1.03 times
+//   heads     N16   6 rounds of 64-channel heads, 16 steps 1.18 times; 3 rounds 0.96
+//             N32   3 rounds 16 steps 1.18; 9 rounds 0.92
+//             N64   1 round 16 steps 1.10; 4.5 rounds 8 steps 1.12, 16 steps 0.92
+//             N128  1 round 8 steps 1.13, 16 steps 0.98; 12 rounds 32 steps 1.03
+int valu_steps(int mode, int N, double r) {
+    if (mode == kModeChannel) {
+        if (N == 16) return steps_at({{1.5, 16}, {4, 8}, {16, 12}, {30, 8}, {45, 24}, {kAnyRounds, 100}}, r);
+        if (N == 32) return steps_at({{1.5, 12}, {3, 4}, {4, 8}, {7, 2}, {8.5, 4}, {11, 2}, {15.5, 4}}, r);
+        if (N == 64) return steps_at({{1, 12}, {1.5, 8}}, r);
+        return steps_at({{2, 0}, {3.9, 8}}, r);
+    }
+    if (N == 16) return steps_at({{2, 16}, {3.9, 12}, {kAnyRounds, 16}}, r);
+    if (N == 32) return steps_at({{1, 16}, {2, 12}, {3.9, 16}, {4.2, 10}, {kAnyRounds, 16}}, r);
+    if (N == 64) return steps_at({{3, 16}, {20, 10}, {kAnyRounds, 16}}, r);
+    return steps_at({{2, 12}, {3, 16}, {7, 8}, {10, 16}, {kAnyRounds, 32}}, r);
+}
+
+// mode channel or head; fast: what mfma_scan_kernel and scan_kernel take but for
+// the row length
+template <int MODE>
+hipError_t launch_scan(const ScanArgs &a, int N, bool fast, hipStream_t st) {
+    if (!fast) return launch_generic<MODE>(a, N, st);
+    const int64_t row = std::max(a.x_row, a.bc_row);
+    const double r = (double)a.B * a.H * (a.P / 16) / device_cus();
+    const bool wide = row >= kMfmaMaxRow;
+    if (a.H <= 65535 && (wide || a.L <= valu_steps(MODE, N, r))) return launch_valu_scan<MODE>(a, N, st);   // (heads along y)
+    if (wide) return launch_generic<MODE>(a, N, st);
+    MfmaScanArgs m{};
+    m.x = a.x; m.b = a.bsrc; m.c = a.csrc; m.decay = a.decay; m.y = a.y; m.chunk_states = a.chunk_states; m.h_in = a.h_in; m.h_out = a.h_out;
+    m.x_row = a.x_row; m.bc_row = a.bc_row; m.B = a.B; m.L = a.L; m.D = a.H * a.P; m.P = a.P; m.cs = a.cs; m.nchunks_out = a.nchunks_out;
+    return launch_mfma_scan(MODE == kModeChannel ? kMScanChannel : kMScanHead, N, m, st);
+}
+
+bool fast_shape(int N, int P, int k, int mode) {
     if (N != 16 && N != 32 && N != 64 && !(N == 128 && mode != kModeModel)) return false;
-    if (P % 16 != 0) return false;
-    return k == 15 && row < kMfmaMaxRow;
+    return P % 16 == 0 && k == 15;
 }
 
 // ------------------------------------------------ float-compat reference
@@ -410,7 +744,7 @@ extern "C" mi_status mi_dyadic_scan(const int8_t *x, const int8_t *b, const int8
     ScanArgs a{};
     a.x = x; a.bsrc = b; a.csrc = c; a.decay = decay_num; a.y = y; a.h_in = h_in; a.h_out = h_out;
     a.x_row = d; a.bc_row = nstate; a.B = batch; a.L = len; a.H = 1; a.P = d; a.k = decay_shift;
-    const bool fast = len > 0 && fast_shape(nstate, d, decay_shift, kModeChannel, d) && aligned(x, 16) && aligned(b, 16) &&
+    const bool fast = len > 0 && fast_shape(nstate, d, decay_shift, kModeChannel) && aligned(x, 16) && aligned(b, 16) &&
                       aligned(c, 16) && aligned(y, 16);
     if (len == 0 && !h_out) return MI_OK;
     hipError_t e = launch_scan<kModeChannel>(a, nstate, fast, as_stream(stream));
@@ -438,7 +772,7 @@ extern "C" mi_status mi_ssd_chunked_scan(const int8_t *x, const int8_t *b, const
     a.x_row = (int64_t)heads * head_dim; a.bc_row = (int64_t)heads * nstate;
     a.B = batch; a.L = len; a.H = heads; a.P = head_dim; a.k = decay_shift;
     a.cs = chunk; a.nchunks_out = (len + chunk - 1) / chunk;
-    const bool fast = len > 0 && fast_shape(nstate, head_dim, decay_shift, kModeHead, (int64_t)heads * (head_dim > nstate ? head_dim : nstate)) && (chunk % kTC == 0) && aligned(x, 16) &&
+    const bool fast = len > 0 && fast_shape(nstate, head_dim, decay_shift, kModeHead) && (chunk % kTC == 0) && aligned(x, 16) &&
                       aligned(b, 16) && aligned(c, 16) && aligned(y, 16);
     hipError_t e = launch_scan<kModeHead>(a, nstate, fast, as_stream(stream));
     if (e != hipSuccess) return fail(MI_ERR_HIP, "mi_ssd_chunked_scan: launch failed: %s", hipGetErrorString(e));
@@ -466,15 +800,15 @@ extern "C" mi_status mi_block_scan(const int8_t *xs, const int8_t *dm, const int
     a.yo = yo; a.h_in = h_in; a.h_out = h_out;
     a.x_row = d_inner; a.bc_row = xp_stride; a.z_row = z_stride;
     a.B = batch; a.L = len; a.H = 1; a.P = d_inner; a.k = decay_shift; a.s_y = s_y;
-    const bool fast = len > 0 && fast_shape(nstate, d_inner, decay_shift, kModeModel, z_stride > xp_stride ? z_stride : xp_stride) && aligned(xs, 16) && aligned(dm, 16) &&
+    const bool fast = len > 0 && fast_shape(nstate, d_inner, decay_shift, kModeModel) && aligned(xs, 16) && aligned(dm, 16) &&
                       aligned(a.z, 16) && aligned(a.bsrc, 16) && aligned(a.csrc, 16) && aligned(yo, 16) &&
                       xp_stride % 16 == 0 && z_stride % 16 == 0;
     hipError_t e;
-    if (fast && nstate != 128)
+    if (fast)
         e = launch_model_scan(xs, dm, a.z, a.bsrc, a.csrc, base, yo, h_in, h_out, d_inner, z_stride, xp_stride, batch,
                               len, d_inner, nstate, s_y, as_stream(stream));
     else
-        e = launch_scan<kModeModel>(a, nstate, fast, as_stream(stream));
+        e = launch_generic<kModeModel>(a, nstate, as_stream(stream));
     if (e != hipSuccess) return fail(MI_ERR_HIP, "mi_block_scan: launch failed: %s", hipGetErrorString(e));
     return MI_OK;
 }
