@@ -1883,7 +1883,13 @@ hipError_t launch_gemm_kind(const GemmArgs &g, hipStream_t st) {
     }
     const int64_t ring = (int64_t)((g.M + kRingBM - 1) / kRingBM) * ((g.N + kRingBN - 1) / kRingBN);
     const int out_unit = kInt8Out ? 16 : 4;
-    if (ring_fits(g, ring) && g.ldo % out_unit == 0 && aligned(g.out, 16)) {
+    // from three of its blocks a CU on, where the 128 x 128 tiles are one round, those
+    // tiles are the faster ones for the epilogues that only store (1000 x 1536 ->
+    // 4096, 1024 tiles, INT8 13.0 against 11.5 us, INT32 15.0 / 14.0; 1500 x 1024 ->
+    // 2048, 768 tiles, 8.2 / 8.8; RESIDUAL at 1024 tiles 16.5 / 18.2, FLOAT 15.7 / 16.9)
+    const bool one_round = (kInt8Out || KIND == MI_OUT_INT32) && g.K >= 1024 && ring > 3 * (int64_t)device_cus() &&
+                           (int64_t)grid.x <= device_cus();
+    if (!one_round && ring_fits(g, ring) && g.ldo % out_unit == 0 && aligned(g.out, 16)) {
         hipLaunchKernelGGL(gemm_ring_kernel<KIND>, dim3((unsigned)ring), dim3(256), 0, st, g);
         return hipGetLastError();
     }
