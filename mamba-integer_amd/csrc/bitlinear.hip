@@ -1762,7 +1762,8 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const float *x, int8_t *
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
     __syncthreads();
     const RowQuant q(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
-    for (int k = threadIdx.x; k < ld; k += 256) xq[row * ld + k] = k < K ? q(xr[k]) : (int8_t)0;
+    for (int k = threadIdx.x; k < K; k += 256) xq[row * ld + k] = q(xr[k]);
+    for (int k = K + threadIdx.x; k < ld; k += 256) xq[row * ld + k] = 0;
     if (threadIdx.x == 0) x_scale[row] = q.x_scale;
 }
 
