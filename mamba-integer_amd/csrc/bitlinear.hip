@@ -1839,7 +1839,6 @@ bool gemm32_fits(const GemmArgs &g, int64_t tiles) {
 // conv 14.4 -> 15.4; 1536 deep 1020 tiles 22.6 -> 18.1, 1536 tiles 25.1 ->
 // 24.9; 2048 deep 528 tiles 20.0 -> 16.1, 784 tiles 15.0 -> 16.6; 4096 deep
 // 1024 tiles 32.9 -> 33.7.
-constexpr int kCus = 256;
 constexpr int64_t kRingMaxTiles = 1152, kRingMaxWork = 1024 * 1536;
 bool ring_fits(const GemmArgs &g, int64_t tiles) {
     return g.K > 0 && g.K % kG2BK == 0 && g.N % 32 == 0 && aligned(g.a, 16) && g.lda % 16 == 0 && aligned(g.w, 16) &&
@@ -1862,11 +1861,11 @@ hipError_t launch_gemm_kind(const GemmArgs &g, hipStream_t st) {
         // 32 (32768 rows 19.2, 16.4, 17.3; 64-row blocks run one a CU)
         if (g.N <= 160 && g.M > 64 && (g.M + 63) / 64 <= 65535 && g.kw % 16 == 0 && g.kw / 16 <= 8 &&
             aligned(g.w, 16) && aligned(g.a, 16) && g.lda % 16 == 0) {
-            const int cols = (g.N + 79) / 80;
+            const int cols = (g.N + 79) / 80, cus = device_cus();
             auto rows = [&](int r) { return (g.M + r - 1) / r; };
-            if (cols * rows(16) <= kCus)
+            if (cols * rows(16) <= cus)
                 hipLaunchKernelGGL((gemv64s_kernel<KIND, 5, 1>), dim3((unsigned)cols, (unsigned)rows(16)), dim3(256), 0, st, g);
-            else if (cols * rows(32) <= kCus || (cols * rows(64) > kCus && rows(32) <= 65535))
+            else if (cols * rows(32) <= cus || (cols * rows(64) > cus && rows(32) <= 65535))
                 hipLaunchKernelGGL((gemv64s_kernel<KIND, 5, 2>), dim3((unsigned)cols, (unsigned)rows(32)), dim3(256), 0, st, g);
             else
                 hipLaunchKernelGGL((gemv64s_kernel<KIND, 5, 4>), dim3((unsigned)cols, (unsigned)rows(64)), dim3(256), 0, st, g);
