@@ -81,19 +81,24 @@ class BitLinear(nn.Module):
         """The packed ternary weights with k padded to a multiple of ``unit`` (16: the
         packing unit, the width of ``forward_int``'s rows; 64: four packed words,
         which the kernels read at once), and their scale; kept per weight version.
-        The key and its packings (by padded k) are replaced as one object, so a
-        call that packs for another key in between leaves this one's alone."""
-        key = (self.weight._version, self.weight.data_ptr(), str(device))
+        The key and its packings are replaced as one object, so a call that packs
+        for another key in between leaves this one's alone; units that pad k alike
+        share a packing."""
+        key = (self.weight._version, self.weight.data_ptr(), device)
         held = self._packed
         if held[0] != key:
             held = self._packed = (key, {})
-        kp = _ceil(self.in_features, unit)
-        if kp not in held[1]:
-            w_quant, w_scale = weight_quant_ternary(self.weight.detach().to("cpu", torch.float32))
-            wq = torch.zeros((self.out_features, kp), dtype=torch.int8)
-            wq[:, : self.in_features] = w_quant.to(torch.int8)
-            held[1][kp] = ops.pack_ternary(wq.to(device)), float(w_scale)
-        return held[1][kp]
+        packed = held[1].get(unit)
+        if packed is None:
+            kp = _ceil(self.in_features, unit)
+            packed = next((p for u, p in list(held[1].items()) if _ceil(self.in_features, u) == kp), None)
+            if packed is None:
+                w_quant, w_scale = weight_quant_ternary(self.weight.detach().to("cpu", torch.float32))
+                wq = torch.zeros((self.out_features, kp), dtype=torch.int8)
+                wq[:, : self.in_features] = w_quant.to(torch.int8)
+                packed = ops.pack_ternary(wq.to(device)), float(w_scale)
+            held[1][unit] = packed
+        return packed
 
     @torch.no_grad()
     def get_ternary_weights(self) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -113,8 +118,8 @@ class BitLinear(nn.Module):
         bias = self.bias
         # one float32 value a feature on the device is added by the GEMM's epilogue,
         # any other bias by torch (with its promotion and broadcasting)
-        fused = (bias is not None and bias.shape == (self.out_features,) and bias.dtype == torch.float32
-                 and bias.device == x.device and bias.is_contiguous())
+        fused = (bias is not None and bias.dim() == 1 and bias.numel() == self.out_features
+                 and bias.dtype == torch.float32 and bias.device == x.device and bias.is_contiguous())
         y = ops.bitlinear_f32(x2, packed, w_scale, bias=bias if fused else None)
         if bias is not None and not fused:
             y = y + bias.to(y.device)
