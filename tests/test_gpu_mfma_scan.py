@@ -1,9 +1,11 @@
 """The scans with their output on the matrix cores against the CPU oracle (bit
-for bit) where their splits and chunks can go wrong: every state count and block
-width of the dispatch (one round of 16-channel blocks, then wider ones), last
-blocks that are partly empty, lengths around the group of four steps and the
-16-, 32- and 64-step chunks, the whole int32 state range, decays 0 and 2^15, bytes
-of -128, and the state handed on."""
+for bit) where their splits and chunks can go wrong: every state count, 16-channel
+blocks and wider ones, last blocks that are partly empty, lengths around the group
+of four steps and the 16-, 32- and 64-step chunks, the whole int32 state range,
+decays 0 and 2^15, bytes of -128, and the state handed on.  (The shortest lengths
+take the VALU kernels; test_gpu_scan_routes.py has both sides of that bound, the
+48-channel blocks of the plain-channel layout and the requant shifts of wide
+blocks.)"""
 
 import numpy as np
 import pytest

@@ -42,12 +42,12 @@ def test_scan_config1_bit_exact(cuda):
 @pytest.mark.parametrize("B,L,D,N", [
     (2, 100, 64, 16), (1, 1, 16, 16), (3, 130, 48, 32), (2, 65, 128, 64),
     (1, 200, 32, 128), (1, 50, 40, 16), (2, 33, 32, 8), (1, 19, 16, 5),
-    # the lane split G follows the channel count B*D at N = 16: 65536 channels
-    # give G = 1, 32768 G = 2, 16384 G = 4, 8192 G = 8, fewer G = 16
+    # many channels: the VALU kernel of short calls at one and two lanes a channel
+    # (65536 and 32768 channels), 16- and 32-channel blocks of the MFMA scan
     (2, 9, 32768, 16), (1, 11, 32768, 16), (1, 13, 16384, 16), (1, 21, 8192, 16), (2, 77, 64, 16),
 ])
 def test_scan_shapes(cuda, B, L, D, N):
-    """Fast kernel at every lane split, ragged D (generic path), odd N, odd L."""
+    """Fast kernels, ragged D (generic path), odd N, odd L."""
     from mamba_int import ops
     rng = np.random.default_rng(B * 1000 + L * 10 + D + N)
     x, b, c, n = _scan_inputs(rng, B, L, D, N)

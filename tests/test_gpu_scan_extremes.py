@@ -154,12 +154,10 @@ def test_ssd_block_scan_state_extremes(cuda, L):
 
 @pytest.mark.parametrize("B,L,D", [(8, 77, 1520), (8, 77, 1552), (1, 33, 8208), (3, 5, 3072)])
 def test_block_scan_mixed_route_edges(cuda, B, L, D):
-    """mi_block_scan from a zero state (no h_in) at the edges of the mixed
-    48-channel block's route (batch x d_inner > 8192 and batch x
-    ceil(d_inner / 48) <= 256): 8 x 1520 ends in a block whose 16-lane half
-    has no channel, 8 x 1552 needs 264 blocks and keeps 8 lanes a channel,
-    1 x 8208 runs 171 mixed blocks, 3 x 3072 192 of them; L not a multiple
-    of 4 or 64."""
+    """mi_block_scan from a zero state (no h_in) around the 48-channel blocks'
+    route (one round of them where 16-channel blocks make three): 8 x 1520 ends
+    in a block with a third of its channels, 8 x 1552 needs 264 blocks, 1 x 8208
+    runs 171, 3 x 3072 192; L not a multiple of 4 or 64."""
     import torch
     from mamba_int import ops
     rng = np.random.default_rng(B * L + D)

@@ -22,13 +22,15 @@ def i32(rng, *shape):
     return rng.integers(-2**31, 2**31, size=shape, dtype=np.int64).astype(np.int32)
 
 
-# rounds below 1, to 1.5 and to 2 (d not a multiple of the block), 48-channel blocks (8192 < b * d <= 12288,
-# also with a partly empty last block), 7 and 34 rounds
-@pytest.mark.parametrize("n,b,d,lengths", [(16, 2, 80, (16, 17)), (16, 3, 2064, (8, 9)), (16, 4, 2064, (33, 70)),
+# from below one round up (d not a multiple of the block), every lane split of the VALU
+# kernel; lengths with every remainder of the MFMA kernel's groups; 48-channel blocks
+# (8192 < b * d <= 12288, also with a partly empty last block)
+@pytest.mark.parametrize("n,b,d,lengths", [(16, 2, 80, (16, 17, 19, 22, 31, 63, 68)), (16, 3, 2064, (8, 9)), (16, 4, 2064, (8, 33, 70)),
                                            (16, 4, 2080, (33, 70)), (16, 7, 4096, (12, 13)), (16, 34, 4112, (24, 25)), (16, 50, 4096, (100,)),
-                                           (32, 2, 80, (12, 13)), (32, 5, 2064, (4, 5)), (32, 7, 2064, (8, 9)),
-                                           (64, 2, 80, (12, 13)), (64, 3, 2048, (8, 9)), (64, 5, 2064, (1, 2)),
-                                           (128, 2, 80, (1, 9)), (128, 6, 2064, (8, 9))])
+                                           (32, 2, 80, (12, 13, 18, 23, 35)), (32, 5, 2064, (4, 5)), (32, 7, 2064, (8, 9)),
+                                           (32, 6, 4096, (2, 3)), (32, 8, 4096, (4, 5)),
+                                           (64, 2, 80, (12, 13, 18, 23, 35)), (64, 3, 2048, (8, 9)), (64, 5, 2064, (1, 2)),
+                                           (128, 2, 80, (1, 9, 15, 18, 35)), (128, 6, 2064, (8, 9))])
 def test_channel_routes(cuda, n, b, d, lengths):
     from mamba_int import ops
     rng = np.random.default_rng(n + b + d)
@@ -41,8 +43,11 @@ def test_channel_routes(cuda, n, b, d, lengths):
         assert np.array_equal(y.cpu().numpy(), y_ref) and np.array_equal(ht.cpu().numpy(), h_ref), length
 
 
-@pytest.mark.parametrize("n,b,heads,p,lengths", [(16, 2, 3, 48, (16, 17)), (16, 8, 24, 64, (12, 13)), (32, 2, 3, 48, (16, 17)),
-                                                 (32, 8, 24, 64, (16, 17)), (64, 2, 5, 16, (16, 17)), (64, 12, 24, 64, (10, 11)),
+@pytest.mark.parametrize("n,b,heads,p,lengths", [(16, 2, 3, 48, (16, 17, 22, 31, 63)), (16, 8, 24, 64, (12, 13)),
+                                                 (16, 12, 24, 64, (16,)), (16, 24, 24, 64, (16, 17)), (16, 44, 24, 64, (16, 17)),
+                                                 (32, 2, 3, 48, (16, 17, 22, 35)), (32, 8, 24, 64, (16, 17)), (32, 12, 24, 64, (16,)),
+                                                 (32, 24, 24, 64, (16,)), (32, 44, 24, 64, (16, 17)),
+                                                 (64, 2, 5, 16, (16, 17, 22, 35)), (64, 12, 24, 64, (10, 11)), (64, 24, 24, 64, (10, 11)),
                                                  (128, 2, 3, 48, (12, 13)), (128, 8, 24, 64, (16, 17)), (128, 32, 24, 64, (32, 33))])
 def test_head_routes(cuda, n, b, heads, p, lengths):
     import torch
@@ -120,3 +125,18 @@ def test_ssd_routes(cuda, n, b, heads, p, lengths):
         ht = T(h)
         yo = ops.ssd_block_scan(T(xs), T(xp), T(z), d, T(tab), heads, n, 14, h_in=ht, h_out=ht)
         assert np.array_equal(yo.cpu().numpy(), ref) and np.array_equal(ht.cpu().numpy(), h_ref), length
+
+
+@pytest.mark.parametrize("s_y", [0, 14, 20, 30])
+@pytest.mark.parametrize("b,d", [(2, 4080), (4, 2064), (4, 2080)])
+def test_block_shifts_of_wide_blocks(cuda, b, d, s_y):
+    """The requant shift in the 32- and 48-channel blocks (last blocks full and partly empty)."""
+    from mamba_int import ops
+    rng = np.random.default_rng(b + d + s_y)
+    n, r, length = 16, 16, 45
+    xs, dm, z = i8(rng, b, length, d), i8(rng, b, length, d), i8(rng, b, length, 2 * d)
+    xp, base, h = i8(rng, b, length, r + 2 * n), rng.integers(0, 32001, size=(d, n), dtype=np.int32), i32(rng, b, d, n)
+    ref, h_ref = O.block_scan(xs, dm, xp, r, z, d, base, 15, s_y, h_state=h.copy())
+    ht = T(h)
+    yo = ops.block_scan(T(xs), T(dm), T(xp), r, T(z), d, T(base), 15, s_y, h_in=ht, h_out=ht)
+    assert np.array_equal(yo.cpu().numpy(), ref) and np.array_equal(ht.cpu().numpy(), h_ref)

@@ -1,6 +1,6 @@
 """Short sequences of many blocks, which take the scans with y on the VALU or
-16-step chunks, against the CPU oracle bit for bit: both sides of the step and
-block bounds, the state handed on, every state count of that dispatch."""
+16-step chunks, against the CPU oracle bit for bit: the state handed on, every
+state count (test_gpu_scan_routes.py has the bounds of the dispatch)."""
 
 import numpy as np
 import pytest
