@@ -913,9 +913,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 // are gemm32_kernel's; each wave keeps its own copy of its weight words.  Rings
 // of four and six stages (less blocks a CU) measured 2 to 30% slower, 128 x 64
 // and 64 x 128 tiles 5 to 30%, and eight waves splitting k 5 to 25%.
-// 2000 x 1536 -> 768 RESIDUAL 17.0 -> 9.9 us, 2103 x 2048 -> 1024 20.0 -> 16.1,
-// 100 x 1536 -> 768 15.1 -> 7.2; in_proj with conv, 100 rows of 768 -> 3072
-// 12.2 -> 6.7, 1000 rows 13.1 -> 10.0.
+// 2000 x 1536 -> 768 RESIDUAL 17.3 -> 9.2 us, 2103 x 2048 -> 1024 20.3 -> 15.7,
+// 100 x 1536 -> 768 15.4 -> 6.7; in_proj with conv, 100 rows of 768 -> 3072
+// 11.4 -> 5.6, 1000 rows 12.2 -> 8.9.
 // Requires K % 128 == 0, N % 32 == 0 (conv: d_inner % 64 == 0), 16-byte aligned
 // a / w with lda % 16 == 0; rows past M and N as in gemm32_kernel.
 constexpr int kRingBM = 64, kRingBN = 64, kRingStages = 3;
@@ -1113,7 +1113,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void g
 // 16 lq .. of its token, one 16-byte store.  All loads are unconditional from
 // clamped addresses and issued before the first product; words past k are
 // zeroed.  Against gemm_any_kernel's 128 x 128 tiles through LDS: 2000 x 48 ->
-// 1536 5.2 -> 4.3 us, 16384 x 48 -> 1536 13.3 -> 10.7 (26 MB: 2.5 TB/s).
+// 1536 4.5 -> 3.7 us, 16384 x 48 -> 1536 12.3 -> 9.9 (26 MB: 2.6 TB/s).
 template <int KIND>
 __global__ __launch_bounds__(256) void gemm_k64_kernel(GemmArgs g) {
     const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;

@@ -31,15 +31,19 @@
 // waves' partials, saturate, gate, requant, store); they run at a raised wave
 // priority, since a chunk's barrier waits for them.
 //
-// Bound: VALU issue.  At B8 x L2048 x 1536 channels, N16 (one block of 48 channels
-// per CU) 10.1 instructions per update of 64 states (13.6 with y on the VALU) at
-// 71% of the issue cycles; with few channels one block's chain of steps (33 ns a
-// step).  us per launch, y on the VALU against here:
-//   model block   B8 x L2048 x 1536, N16      214 -> 139    B2 x L1000 x 1536   108 -> 38
-//                 B3 x L701 x 2048             78 -> 43      B64 x L512 x 4096   797 -> 759
-//   SSD block     B2 x L1023, 24 x 64, N64    160 -> 73     B8 x L2048          592 -> 393
-//   head layout   B4 x L8192, 24 x 64, N128  2108 -> 1600
-//   channels      B1 x L256 x 512, N16         23 -> 10     B8 x L2048 x 1536   291 -> 116
+// Bound: VALU issue where every CU has a block (B8 x L2048 x 1536 channels, N16, one
+// block of 48 channels a CU: 9.6 instructions per update of 64 states, 13.6 with y on
+// the VALU, at 67% of the issue cycles); the CUs themselves where the blocks are
+// fewer (the head layout below: 192 blocks of 32 channels on 256 CUs, at 74% of the
+// issue cycles of those that work); with few channels one block's chain of steps
+// (33 ns a step).  us per launch alone, y on the VALU against here:
+//   model block   B8 x L2048 x 1536, N16      210 -> 149 (in the model, behind other
+//                                             kernels, 146 to 164)
+//                 B2 x L1000 x 1536           105 -> 37      B3 x L701 x 2048   75 -> 42
+//                 B64 x L512 x 4096           806 -> 778
+//   SSD block     B2 x L1023, 24 x 64, N64    160 -> 71      B8 x L2048        590 -> 392
+//   head layout   B4 x L8192, 24 x 64, N128  2119 -> 1579
+//   channels      B1 x L256 x 512, N16         22 -> 8       B8 x L2048 x 1536 285 -> 111
 #include <stddef.h>
 
 #include <type_traits>
@@ -550,7 +554,7 @@ hipError_t launch(const MfmaScanArgs &a, hipStream_t st) {
 //   N = 16   16-channel blocks of 64-step chunks 33; 32 channels 50 (42 without
 //            the gate); 48 channels 67 (73).  The least rounds x time wins: one
 //            block per CU of 16 channels up to 4096 channels, 32 up to 8192, 48
-//            up to 12288 and beyond (B64 x L512 x 4096 channels: 759 us, 855 with
+//            up to 12288 and beyond (B64 x L512 x 4096 channels: 778 us, 855 with
 //            32-channel blocks).  Up to 256 steps and beyond one round, 32-channel
 //            blocks of 16-step chunks, two resident a CU: a block's start costs as
 //            much as its steps (B16 x L64 x 1536 16.9 -> 15.4 us, B32 x L256 x 4096
@@ -561,7 +565,8 @@ hipError_t launch(const MfmaScanArgs &a, hipStream_t st) {
 //   N = 128  four states a lane; beyond one round of 16-channel blocks 32 channels
 //            (two sets share a lane's C operand; B4 x L8192 x 24 heads of 64: 1600
 //            against 2045 us)
-// Returns hipErrorInvalidValue for a case it does not take (see mfma_scan_takes).
+// Returns hipErrorInvalidValue for a state count it does not take (mfma_scan.hpp has
+// the other conditions; short sequences go to other kernels before this).
 hipError_t launch_mfma_scan(int mode, int N, const MfmaScanArgs &a, hipStream_t st) {
     const int64_t cus = device_cus();
     auto rounds = [&](int ch) { return ((int64_t)a.B * ((a.D + ch - 1) / ch) + cus - 1) / cus; };
