@@ -76,6 +76,12 @@ class BitLinear(nn.Module):
             self.register_parameter("bias", None)
         self._packed = (None, {})
 
+    def __setstate__(self, state):
+        # a saved or copied module packs its own weights (modules saved whole by
+        # earlier versions hold other values here)
+        super().__setstate__(state)
+        self._packed = (None, {})
+
     # ------------------------------------------------------------ weights
     def _packed_weights(self, device, unit: int) -> Tuple[torch.Tensor, float]:
         """The packed ternary weights with k padded to a multiple of ``unit`` (16: the

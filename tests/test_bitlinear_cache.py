@@ -1,6 +1,8 @@
 """BitLinear's packed weights are kept per weight version and device: a pack for
 another device between the key's check and the store (another thread's call)
 reaches neither call's weights, and equal padded widths share one packing."""
+import copy
+
 import pytest
 import torch
 
@@ -49,3 +51,20 @@ def test_equal_widths_share_a_packing(packs, k, count):
     assert layer._packed_weights(torch.device("cpu"), 64)[0].shape[1] == 128
     assert layer._packed_weights(torch.device("cpu"), 16)[0].shape[1] == -(-k // 16) * 16
     assert len(packs) == count
+
+
+@pytest.mark.parametrize("held", [None, {}, {64: (torch.zeros(8, 16, dtype=torch.uint8), 1.0)}], ids=["none", "empty", "packed"])
+def test_module_saved_whole_by_earlier_versions(packs, held):
+    layer = BitLinear(24, 8)
+    state = dict(layer.__dict__, _packed=held, _packed_key=None)
+    loaded = BitLinear.__new__(BitLinear)
+    loaded.__setstate__(state)
+    assert torch.equal(loaded._packed_weights(torch.device("cpu"), 64)[0], layer._packed_weights(torch.device("cpu"), 64)[0])
+
+
+def test_copy_packs_its_own_weights(packs):
+    layer = BitLinear(24, 8)
+    layer._packed_weights(torch.device("cpu"), 64)
+    for other in (copy.copy(layer), copy.deepcopy(layer)):
+        other._packed_weights(torch.device("cpu"), 16)
+        assert set(layer._packed[1]) == {64}
