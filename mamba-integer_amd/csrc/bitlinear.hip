@@ -1875,7 +1875,7 @@ hipError_t launch_gemm_kind(const GemmArgs &g, hipStream_t st) {
     if constexpr (kInt8Out) {
         if (g.K > 0 && g.K <= 64 && g.N % 16 == 0 && g.ldo % 16 == 0 && aligned(g.out, 16)) {
             const int64_t blocks = (int64_t)((g.M + 63) / 64) * ((g.N + 255) / 256);
-            if (blocks <= INT32_MAX) {
+            if (blocks < 1 << 24) {   // (a launch's threads stay below 2^32)
                 hipLaunchKernelGGL(gemm_k64_kernel<KIND>, dim3((unsigned)blocks), dim3(256), 0, st, g);
                 return hipGetLastError();
             }

@@ -10,7 +10,7 @@
 
 dim3 blockIdx, threadIdx, blockDim, gridDim;
 int8_t *host_dynamic_lds;
-int host_vote, host_cus;
+int host_vote, host_cus, host_dry, host_error;
 const char *host_kernel = "";
 
 void host_die(const char *what, long long a, long long b) {
@@ -164,12 +164,25 @@ void decode(int m, int d, int N, int R) {
     call(mi_argmax_i32(p.get<int32_t>((size_t)m * V), V, ids, m, V, nullptr));
 }
 
+// calls at the launch limits, which no kernel runs for: every one has a kernel that takes it
+void limits() {
+    host_dry = 1;
+    host_cus = 256;
+    auto *b = (int8_t *)(1ull << 40);
+    for (int m : {585956566, 586902066})
+        for (int k : {16, 32, 48, 64})
+            for (int kind : {MI_OUT_INT8, MI_OUT_DECAY_MOD})
+                call(mi_bitlinear_gemm(b, k, (uint8_t *)b, b, 352, kind, m, 352, k, 6, 0, 0, 0, nullptr, 1.0f, nullptr, nullptr));
+    if (refused) printf("last kernel %s\n", host_kernel), exit(4);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
     const char *what = argv[1];
     auto is = [&](const char *s) { return !strcmp(what, s); };
     rng.seed(atoi(argv[3]));
+    if (is("limits")) limits();
     for (int i = 0; i < atoi(argv[2]); ++i) {
         host_vote = i & 1;
         // the dispatch of small and of large devices, so that every split is reached at small sizes
@@ -181,6 +194,7 @@ int main(int argc, char **argv) {
         else if (is("ssd_scan")) ssd_scan(logu(1, 8), logu(1, 200), logu(1, 24), 16 * uni(1, 5), 16 << uni(0, 2));
         else if (is("scans")) scans(logu(1, 16), logu(1, 250));
         else if (is("elementwise")) elementwise(logu(1, 64), logu(1, 150), logu(1, 1500));
+        else if (is("limits")) continue;
         else if (is("decode")) decode(logu(1, 70), 64 * logu(1, 10), 16 << uni(0, 2), 16 * uni(1, 5));
         else return 2;
     }

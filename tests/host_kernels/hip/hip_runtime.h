@@ -114,7 +114,8 @@ typedef int hipError_t;
 enum { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorNotReady = 2, hipDeviceAttributeMultiprocessorCount = 0 };
 extern int host_cus;
 inline const char *hipGetErrorString(int) { return "error"; }
-inline int hipGetLastError() { return 0; }
+extern int host_dry, host_error;   // dry: launches are checked against the runtime's limits, not run
+inline int hipGetLastError() { const int e = host_error; host_error = 0; return e; }
 inline int hipGetDevice(int *d) { *d = 0; return 0; }
 inline int hipDeviceGetAttribute(int *v, int, int) { *v = host_cus; return 0; }
 enum { hipMemcpyDeviceToDevice, hipMemcpyHostToDevice };
@@ -125,6 +126,10 @@ extern const char *host_kernel;
 template <class... P, class... A> void host_launch(const char *name, void (*f)(P...), dim3 g, dim3 b, size_t dyn, A... a) {
     host_kernel = name;
     gridDim = g; blockDim = b;
+    if (host_dry) {
+        if (!g.x || (uint64_t)g.x * b.x >> 32 || !g.y || g.y > 65535 || !g.z || g.z > 65535) host_error = hipErrorInvalidValue;
+        return;
+    }
     host_dynamic_lds = dyn ? (int8_t *)aligned_alloc(16, (dyn + 15) / 16 * 16) : nullptr;
     for (unsigned z = 0; z < g.z; ++z) for (unsigned y = 0; y < g.y; ++y) for (unsigned x = 0; x < g.x; ++x) {
         blockIdx = dim3(x, y, z);

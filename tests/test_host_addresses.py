@@ -71,7 +71,8 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("family,count", [("bitlinear", 120), ("bitlinear_f32", 60), ("block", 50), ("block_2103", 1),
-                                          ("ssd_scan", 50), ("scans", 40), ("elementwise", 60), ("decode", 30)])
+                                          ("ssd_scan", 50), ("scans", 40), ("elementwise", 60), ("decode", 30),
+                                          ("limits", 0)])
 def test_addresses_in_bounds(program, family, count):
     out = subprocess.run([program, family, str(count), "1"], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0, (out.stdout + out.stderr)[-6000:]
