@@ -696,7 +696,9 @@ void launch_elem_scan(const int32_t *u, const int32_t *n, int k, int cs, int32_t
     // the chunked form (32768 x 3, 64 steps 27 us, 33 with 256 lanes; elementwise 8192
     // x 100, 16 steps 26 with 64, 21 with 256).
     const int64_t cw = 64 / rows, waves = std::min<int64_t>(B * ((C + cw - 1) / cw), 1 << 20);
-    if (L < (rows == 4 ? 16 : 32) || (2 * (int64_t)C <= cw && (waves * waves * waves) >> (rows == 4 ? 29 : 27) >= L)) {
+    // And for 2^24 sequences and more: a launch has less blocks of 256 lanes than that.
+    if (L < (rows == 4 ? 16 : 32) || B >= 1 << 24 ||
+        (2 * (int64_t)C <= cw && (waves * waves * waves) >> (rows == 4 ? 29 : 27) >= L)) {
         const bool one = L < 4 || (!CHUNKED && L == 4);
         const unsigned threads = one || (!CHUNKED && lanes >= 65536) ? 256 : 64;
         const dim3 grid((unsigned)((lanes + threads - 1) / threads));

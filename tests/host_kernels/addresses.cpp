@@ -168,7 +168,13 @@ void decode(int m, int d, int N, int R) {
 void limits() {
     host_dry = 1;
     host_cus = 256;
-    auto *b = (int8_t *)(1ull << 40);
+    auto *p = (int32_t *)(1ull << 40);
+    auto *b = (int8_t *)p;
+    for (int B : {1 << 24, 16867619, 20000000})
+        for (int C : {33, 36}) {
+            call(mi_dyadic_scan_elementwise(p, p, 15, p, p, p, B, 33, C, nullptr));
+            call(mi_dyadic_chunked_scan(p, p, 15, 12, p, p, p, p, p, B, 33, C, nullptr));
+        }
     for (int m : {585956566, 586902066})
         for (int k : {16, 32, 48, 64})
             for (int kind : {MI_OUT_INT8, MI_OUT_DECAY_MOD})
