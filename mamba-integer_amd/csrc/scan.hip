@@ -688,17 +688,21 @@ void launch_elem_scan(const int32_t *u, const int32_t *n, int k, int cs, int32_t
     // One lane per channel instead for few steps, where the rows' 16 groups ahead are
     // mostly the last one again (rows / lanes, us: 32768 x 64 channels, 1 step 21.7 /
     // 7.1, 16 steps 49.0 / 46.4; 512 x 32, 8 steps 3.1 / 2.7, 16 steps 3.4 / 3.4, 32
-    // steps 4.3 / 4.7), and for sequences that fill half a wave or less, up to a
-    // length that grows with the waves there are (rows / lanes: 2048 of them, 64 steps
-    // 0.9 to 1.04, 256 steps 0.5 to 0.8; 4096, 256 steps 0.85 with four rows, 1.1 to 1.4
-    // with one or two; 8192, 1000 steps 1.14 to 1.9).  Four steps and fewer: one load
-    // ahead (eight repeat the last).  Blocks of 64 lanes where there are few, and in
-    // the chunked form (32768 x 3, 64 steps 27 us, 33 with 256 lanes; elementwise 8192
-    // x 100, 16 steps 26 with 64, 21 with 256).
-    const int64_t cw = 64 / rows, waves = std::min<int64_t>(B * ((C + cw - 1) / cw), 1 << 20);
-    // And for 2^24 sequences and more: a launch has less blocks of 256 lanes than that.
-    if (L < (rows == 4 ? 16 : 32) || B >= 1 << 24 ||
-        (2 * (int64_t)C <= cw && (waves * waves * waves) >> (rows == 4 ? 29 : 27) >= L)) {
+    // steps 4.3 / 4.7), and for sequences that fill half a wave or less where their
+    // waves, several on a SIMD, take longer.  ns a step measured at 1000 steps and more
+    // (rows 4 / 2 / 1, lanes): 1024 sequences of one channel 46 / 56 / 73, 125; 4096 100 /
+    // 135 / 167, 130; 8192 170 / 225 / 285, 135; chunked, 6000 in odd chunks - / - / 305,
+    // 150; a wave's 24 / 32 / 40 each (chunked a quarter more) and the loads of 64 steps
+    // before the first, a lane's chain 140 and the stream of 0.5 for 1024 lanes.  And for
+    // 2^24 sequences and more: a launch has less blocks of 256 lanes than that.
+    // Four steps and fewer: one load ahead (eight repeat the last).  Blocks of 64 lanes
+    // where there are few, and in the chunked form (32768 x 3, 64 steps 27 us, 33 with
+    // 256 lanes; elementwise 8192 x 100, 16 steps 26 with 64, 21 with 256).
+    const int64_t cw = 64 / rows, waves = B * ((C + cw - 1) / cw), simds = 4 * (int64_t)device_cus();
+    const double wave_ns = (rows == 4 ? 24 : rows == 2 ? 32 : 40) * (CHUNKED ? 1.25 : 1.0);
+    const double rows_ns = (double)((waves + simds - 1) / simds) * wave_ns * (L + 64.0);
+    const double lanes_ns = (140 + 0.5 * (double)lanes / 1024) * L;
+    if (L < (rows == 4 ? 16 : 32) || (2 * (int64_t)C <= cw && rows_ns > lanes_ns) || B >= 1 << 24) {
         const bool one = L < 4 || (!CHUNKED && L == 4);
         const unsigned threads = one || (!CHUNKED && lanes >= 65536) ? 256 : 64;
         const dim3 grid((unsigned)((lanes + threads - 1) / threads));

@@ -16,7 +16,8 @@ def T(a):
 
 @pytest.mark.parametrize("b,length,c", [(1, 1, 1), (3, 4, 70), (2, 5, 33), (3, 15, 65), (3, 16, 65), (2, 31, 10300), (2, 32, 10300),
                                         (300, 9, 300), (300, 33, 300), (8200, 17, 1), (4100, 40, 5), (4096, 40, 8), (2048, 17, 8),
-                                        (2049, 33, 16)])
+                                        (2049, 33, 16), (2048, 155, 1), (2048, 160, 1), (4096, 130, 1), (4096, 136, 1),
+                                        (4096, 345, 1), (4096, 355, 1), (6000, 400, 2)])
 def test_elementwise_and_chunked(cuda, b, length, c):
     import torch
     from mamba_int import ops
