@@ -25,6 +25,7 @@
 //                 K; each lane streams 16-byte words of packed weights straight
 //                 from HBM and unpacks them in registers.
 #include <algorithm>
+#include <type_traits>
 
 #include "mi_mfma.hpp"
 
@@ -70,10 +71,11 @@ __device__ __forceinline__ int64_t residual_delta(const GemmArgs &g, int32_t acc
 // where every increment fits 32 bits): one 32 x 32 + 64 multiply-add with the
 // rounding constant, one v_alignbit for the shift, and a saturating 32-bit add
 // in place of the 64-bit shift, add and clamp (6 instructions a value, not
-// ~20; gemm_kernel, 16384 x 1536 -> 768: 38.7 -> 36.9 us).
+// ~20; gemm_kernel, 16384 x 1536 -> 768: 33.4 -> 31.7 us).
+template <bool R32>
 __device__ __forceinline__ v4i residual4(const GemmArgs &g, v4i old, v4i acc) {
     v4i nv;
-    if (g.res32) {
+    if constexpr (R32) {
         const int64_t half = (int64_t)1 << (g.res_shift - 1);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -88,6 +90,20 @@ __device__ __forceinline__ v4i residual4(const GemmArgs &g, v4i old, v4i acc) {
             nv[r] = (int32_t)clamp64((int64_t)old[r] + residual_delta(g, acc[r]), -kResidualLimit, kResidualLimit);
     }
     return nv;
+}
+// (gemm32_kernel chooses at each value: chosen once, its 64-bit form gained 3%, 48.7 ->
+// 47.1 us at 16384 x 2048 -> 1024, and the 32-bit one lost 1.5% at 32768 x 4096 -> 2048)
+__device__ __forceinline__ v4i residual4(const GemmArgs &g, v4i old, v4i acc) {
+    return g.res32 ? residual4<true>(g, old, acc) : residual4<false>(g, old, acc);
+}
+
+// An epilogue for the width of the increment and with or without row statistics.
+template <class F>
+__device__ __forceinline__ void residual_form(const GemmArgs &g, F epilogue) {
+    if (g.res32 && !g.row_stats) epilogue(std::true_type{}, std::false_type{});
+    else if (g.res32) epilogue(std::true_type{}, std::true_type{});
+    else if (!g.row_stats) epilogue(std::false_type{}, std::false_type{});
+    else epilogue(std::false_type{}, std::true_type{});
 }
 
 // INT8 / DECAY_MOD outputs of 4 consecutive features as one dword.
@@ -502,35 +518,41 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const ConvArgs &cv)
                     const int n = n0 + nb + i * 16 + 4 * lq;
                     old[jj][i] = *reinterpret_cast<const v4i *>(ob + (int64_t)m * g.ldo + (n < g.N ? n : 0));
                 }
+            // the width and the statistics of a group's values, chosen here: chosen at each
+            // of them, the 64-bit form with statistics took 14.2 us at 634 x 192 -> 224, here
+            // 11.5, and 40.1 at 16384 x 1536 -> 768, 39.6; the 32-bit one without 34.9, 31.7
+            residual_form(g, [&](auto r32, auto stats) {
+                constexpr bool R32 = decltype(r32)::value, STATS = decltype(stats)::value;
 #pragma unroll
-            for (int jj = 0; jj < JG; ++jj) {
-                const int j = JG * h + jj;
-                const int m = m0 + mb + j * 16 + l16;
-                RowStat st{0, 0};
+                for (int jj = 0; jj < JG; ++jj) {
+                    const int j = JG * h + jj;
+                    const int m = m0 + mb + j * 16 + l16;
+                    RowStat st{0, 0};
 #pragma unroll
-                for (int i = 0; i < NI; ++i) {
-                    const int n = n0 + nb + i * 16 + 4 * lq;
-                    if (m < g.M && n < g.N) {
-                        const v4i nv = residual4(g, old[jj][i], acc[i][j]);
-                        int32_t *o = ob + (int64_t)m * g.ldo + n;
-                        if (n + 3 < g.N) {
-                            *reinterpret_cast<v4i *>(o) = nv;
-                        } else {
-                            for (int r = 0; r < 4 && n + r < g.N; ++r) o[r] = nv[r];
-                        }
-                        if (g.row_stats) {
+                    for (int i = 0; i < NI; ++i) {
+                        const int n = n0 + nb + i * 16 + 4 * lq;
+                        if (m < g.M && n < g.N) {
+                            const v4i nv = residual4<R32>(g, old[jj][i], acc[i][j]);
+                            int32_t *o = ob + (int64_t)m * g.ldo + n;
+                            if (n + 3 < g.N) {
+                                *reinterpret_cast<v4i *>(o) = nv;
+                            } else {
+                                for (int r = 0; r < 4 && n + r < g.N; ++r) o[r] = nv[r];
+                            }
+                            if constexpr (STATS) {
 #pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                if (n + r < g.N) {
-                                    st.s1 += nv[r];
-                                    st.s2 += (int64_t)nv[r] * nv[r];
+                                for (int r = 0; r < 4; ++r) {
+                                    if (n + r < g.N) {
+                                        st.s1 += nv[r];
+                                        st.s2 += (int64_t)nv[r] * nv[r];
+                                    }
                                 }
                             }
                         }
                     }
+                    if constexpr (STATS) flush_row_stat(g, st, m, lq);
                 }
-                if (g.row_stats) flush_row_stat(g, st, m, lq);
-            }
+            });
         }
     } else {
 #pragma unroll
@@ -1886,7 +1908,7 @@ hipError_t launch_gemm_kind(const GemmArgs &g, hipStream_t st) {
     // from three of its blocks a CU on, where the 128 x 128 tiles are one round, those
     // tiles are the faster ones for the epilogues that only store (1000 x 1536 ->
     // 4096, 1024 tiles, INT8 13.0 against 11.5 us, INT32 15.0 / 14.0; 1500 x 1024 ->
-    // 2048, 768 tiles, 8.2 / 8.8; RESIDUAL at 1024 tiles 16.5 / 18.2, FLOAT 15.7 / 16.9)
+    // 2048, 768 tiles, 8.2 / 8.8; RESIDUAL at 1024 tiles 16.4 / 16.8, FLOAT 15.7 / 16.9)
     const bool one_round = (kInt8Out || KIND == MI_OUT_INT32) && g.K >= 1024 && ring > 3 * (int64_t)device_cus() &&
                            (int64_t)grid.x <= device_cus();
     if (!one_round && ring_fits(g, ring) && g.ldo % out_unit == 0 && aligned(g.out, 16)) {
