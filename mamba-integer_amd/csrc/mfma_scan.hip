@@ -46,7 +46,9 @@
 //   channels      B1 x L256 x 512, N16         22 -> 8       B8 x L2048 x 1536 285 -> 111
 #include <stddef.h>
 
+#include <initializer_list>
 #include <type_traits>
+#include <utility>
 
 #include "mfma_scan.hpp"
 #include "mi_mfma.hpp"
@@ -548,54 +550,115 @@ hipError_t launch(const MfmaScanArgs &a, hipStream_t st) {
 
 }  // namespace
 
-
-// Which split, by the blocks of 16, 32 and 48 channels that the call makes (us
+// Channels of a block, by the blocks of 16, 32 and 48 channels that the call makes (us
 // per 1000 steps measured with one block on every CU):
 //   N = 16   16-channel blocks of 64-step chunks 33; 32 channels 50 (42 without
 //            the gate); 48 channels 67 (73).  The least rounds x time wins: one
 //            block per CU of 16 channels up to 4096 channels, 32 up to 8192, 48
 //            up to 12288 and beyond (B64 x L512 x 4096 channels: 778 us, 855 with
-//            32-channel blocks).  Up to 256 steps and beyond one round, 32-channel
-//            blocks of 16-step chunks, two resident a CU: a block's start costs as
-//            much as its steps (B16 x L64 x 1536 16.9 -> 15.4 us, B32 x L256 x 4096
-//            205 -> 193, B64 x L128 x 4096 234 -> 204).
+//            32-channel blocks).
 //   N = 32   two states a lane; the model's 48-channel blocks beyond one round of
 //            16 (B8 x L200 x 1536 channels 32.8 against 34.9 us, B32 115 / 114)
 //   N = 64   four states a lane (two: B8 x L1000 x 1536 channels 200 against 174 us)
 //   N = 128  four states a lane; beyond one round of 16-channel blocks 32 channels
 //            (two sets share a lane's C operand; B4 x L8192 x 24 heads of 64: 1600
-//            against 2045 us)
+//            against 2045 us), in heads that they divide
+static int block_channels(int mode, int N, int B, int D, int P) {
+    const int64_t cus = device_cus();
+    auto rounds = [&](int ch) { return ((int64_t)B * ((D + ch - 1) / ch) + cus - 1) / cus; };
+    const int64_t r16 = rounds(16), r32 = rounds(32), r48 = rounds(48);
+    if (N == 16 && (mode == kMScanModel || mode == kMScanChannel)) {
+        const int64_t t32 = mode == kMScanModel ? 50 : 42, t48 = mode == kMScanModel ? 67 : 73;
+        if (33 * r16 <= t32 * r32 && 33 * r16 <= t48 * r48) return 16;
+        return t32 * r32 <= t48 * r48 ? 32 : 48;
+    }
+    if (N == 32 && mode == kMScanModel) return r16 <= 1 ? 16 : 48;
+    if (N == 128) return r16 <= 1 || (mode == kMScanHead && P % 32) ? 16 : 32;
+    return 16;
+}
+
+// A block of the MFMA scan starts slower than one of the VALU kernels (tables, five
+// waves' first loads, the helpers' barriers) and its rounds are whole, so short
+// sequences are faster there, and with several blocks a CU some of any length.  The
+// steps up to which they were, by rounds: the blocks' channels in sixteens over CUs, to
+// the next whole block.  Taken from 71,000 random sizes of 2 to 500 steps, both
+// kernels each: 0.4% are slower by more than 4% than on the VALU kernels alone (one
+// table over channels, not whole blocks, left 2.9%, up to 1.9 times).  MFMA / VALU, us:
+//   model N16   6 x 42 x 2048 (batch x steps x channels) 16.8 / 10.2, 31 x 41 x 784 31.7 /
+//               14.0, 8 x 512 x 1536 43 / 63, 53 x 269 x 3264 362 / 308 (14 rounds of 48)
+//         N32   12 x 38 x 1024 20.7 / 12.4, 59 x 494 x 400 211 / 161; N64 beyond two rounds
+//   heads N64   55 x 17 x 54 of 128 206 / 113, 53 x 374 x 5 of 32 65 / 115
+//         N32   57 x 21 x 52 of 128 157 / 108; N128 22 x 18 x 21 of 48 35.2 / 29.0
+//   channels    N16 64 x 16 x 4096 54 / 39, 1 x 32 x 4096 4.7 / 5.1
+int valu_scan_steps(int mode, int N, int B, int D, int P) {
+    const int ch = block_channels(mode, N, B, D, P);
+    const double r = (double)B * ((D + ch - 1) / ch) * (ch / 16) / device_cus();
+    constexpr double kRest = 1e30;
+    constexpr int kAll = INT32_MAX;
+    auto steps = [&](std::initializer_list<std::pair<double, int>> table) {   // (rounds up to, steps)
+        for (const auto &e : table)
+            if (r <= e.first) return e.second;
+        return 0;
+    };
+    if (mode == kMScanChannel) {
+        if (N == 16 && ch == 16) return steps({{1, 16}, {kRest, 64}});
+        if (N == 16 && ch == 32) return steps({{6, 16}, {8, 24}, {12, 12}, {16, 28}, {21, 4}, {kRest, 24}});
+        if (N == 16) return 12;
+        if (N == 32) return steps({{2, 14}, {3, 4}, {4, 22}, {6, 2}, {8, 12}, {10, 0}, {16, 8}});
+        if (N == 64) return steps({{1, 14}, {2, 6}, {3, 0}, {4, 6}, {6, 0}, {8, 6}});
+        return ch == 16 ? 0 : steps({{2, 4}, {4, 14}});
+    }
+    if (mode == kMScanHead) {
+        if (N == 16) return steps({{3, 14}, {4, 28}, {5.5, 16}, {8, 28}, {11, 18}, {16, 24}, {21, 14}, {39, 18}, {kRest, 32}});
+        if (N == 32) return steps({{2, 14}, {4, 24}, {12, 14}, {16, 20}, {27, 10}, {kRest, 24}});
+        if (N == 64) return steps({{1, 28}, {4, 18}, {6, 12}, {8, 20}, {13, 10}, {23, 14}, {45, 18}, {kRest, 40}});
+        if (ch == 16) return steps({{1, 18}, {2, 64}, {5.5, 20}, {9, 14}, {kRest, 36}});
+        return steps({{2, 14}, {4, 28}, {6, 10}, {10, 18}, {21, 28}, {kRest, 40}});
+    }
+    if (mode == kMScanModel) {
+        if (N == 16 && ch == 16) return steps({{1, 2}, {kRest, 128}});
+        if (N == 16 && ch == 32) return steps({{2, 14}, {6, 40}, {14, 64}, {kRest, kAll}});
+        if (N == 16) return steps({{4.5, 24}, {6, 40}, {18, 64}, {57, kAll}, {kRest, 128}});
+        if (N == 32 && ch == 16) return 4;
+        if (N == 32) return steps({{2, kAll}, {3, 24}, {4, kAll}, {4.5, 160}, {6, 80}, {8, kAll}, {9, 64}, {kRest, kAll}});
+        return steps({{1, 28}, {2, 160}, {kRest, kAll}});
+    }
+    if (N == 16) return steps({{1, 0}, {2, 6}, {3, 12}, {10, 40}, {kRest, 64}});
+    if (N == 32) return steps({{1, 2}, {2, 10}, {3, 28}, {5, 48}, {kRest, 64}});
+    return steps({{1, 18}, {7, 64}, {kRest, 128}});
+}
+
+// The model's 32- and 48-channel blocks of N = 16 run up to 256 steps, beyond one round,
+// as 32-channel blocks of 16-step chunks, two resident a CU: a block's start costs as
+// much as its steps (B16 x L64 x 1536 16.9 -> 15.4 us, B32 x L256 x 4096 205 -> 193,
+// B64 x L128 x 4096 234 -> 204).
 // Returns hipErrorInvalidValue for a state count it does not take (mfma_scan.hpp has
 // the other conditions; short sequences go to other kernels before this).
 hipError_t launch_mfma_scan(int mode, int N, const MfmaScanArgs &a, hipStream_t st) {
-    const int64_t cus = device_cus();
-    auto rounds = [&](int ch) { return ((int64_t)a.B * ((a.D + ch - 1) / ch) + cus - 1) / cus; };
-    const int64_t r16 = rounds(16), r32 = rounds(32), r48 = rounds(48);
+    const int ch = block_channels(mode, N, a.B, a.D, a.P);
+    const bool one16 = (int64_t)a.B * ((a.D + 15) / 16) <= device_cus();
     if (mode == kMScanModel) {
         if (N == 16) {
-            if (33 * r16 <= 50 * r32 && 33 * r16 <= 67 * r48) return launch<kMScanModel, 16, 1, 1, 1, 64>(a, st);
-            if (r48 > 1 && a.L <= 256) return launch<kMScanModel, 16, 1, 1, 2, 16>(a, st);
-            if (50 * r32 <= 67 * r48) return launch<kMScanModel, 16, 1, 1, 2, 32>(a, st);
-            return launch<kMScanModel, 16, 1, 1, 3, 32>(a, st);
+            if (ch == 16) return launch<kMScanModel, 16, 1, 1, 1, 64>(a, st);
+            if (a.L <= 256 && (int64_t)a.B * ((a.D + 47) / 48) > device_cus()) return launch<kMScanModel, 16, 1, 1, 2, 16>(a, st);
+            return ch == 32 ? launch<kMScanModel, 16, 1, 1, 2, 32>(a, st) : launch<kMScanModel, 16, 1, 1, 3, 32>(a, st);
         }
-        if (N == 32) return r16 <= 1 ? launch<kMScanModel, 32, 2, 1, 1, 32>(a, st) : launch<kMScanModel, 32, 2, 1, 3, 32>(a, st);
+        if (N == 32) return ch == 16 ? launch<kMScanModel, 32, 2, 1, 1, 32>(a, st) : launch<kMScanModel, 32, 2, 1, 3, 32>(a, st);
         if (N == 64) return launch<kMScanModel, 64, 2, 1, 1, 32>(a, st);
     } else if (mode == kMScanChannel) {
-        if (N == 16) {
-            if (33 * r16 <= 42 * r32 && 33 * r16 <= 73 * r48) return launch<kMScanChannel, 16, 1, 1, 1, 64>(a, st);
-            if (42 * r32 <= 73 * r48) return launch<kMScanChannel, 16, 1, 1, 2, 32>(a, st);
-            return launch<kMScanChannel, 16, 1, 1, 3, 32>(a, st);
-        }
+        if (N == 16)
+            return ch == 16   ? launch<kMScanChannel, 16, 1, 1, 1, 64>(a, st)
+                   : ch == 32 ? launch<kMScanChannel, 16, 1, 1, 2, 32>(a, st)
+                              : launch<kMScanChannel, 16, 1, 1, 3, 32>(a, st);
         if (N == 32) return launch<kMScanChannel, 32, 2, 1, 1, 32>(a, st);
         if (N == 64) return launch<kMScanChannel, 64, 4, 1, 1, 32>(a, st);
-        if (N == 128) return r16 <= 1 ? launch<kMScanChannel, 128, 4, 1, 1, 16>(a, st) : launch<kMScanChannel, 128, 4, 2, 1, 16>(a, st);
+        if (N == 128) return ch == 16 ? launch<kMScanChannel, 128, 4, 1, 1, 16>(a, st) : launch<kMScanChannel, 128, 4, 2, 1, 16>(a, st);
     } else if (mode == kMScanHead) {
         // (a block lies in one head: more than 16 channels only where they divide it)
-        if (N == 16) return r16 <= 1 ? launch<kMScanHead, 16, 1, 1, 1, 64>(a, st) : launch<kMScanHead, 16, 1, 1, 1, 32>(a, st);
+        if (N == 16) return one16 ? launch<kMScanHead, 16, 1, 1, 1, 64>(a, st) : launch<kMScanHead, 16, 1, 1, 1, 32>(a, st);
         if (N == 32) return launch<kMScanHead, 32, 2, 1, 1, 32>(a, st);
         if (N == 64) return launch<kMScanHead, 64, 4, 1, 1, 32>(a, st);
-        if (N == 128)
-            return r16 <= 1 || a.P % 32 ? launch<kMScanHead, 128, 4, 1, 1, 16>(a, st) : launch<kMScanHead, 128, 4, 2, 1, 16>(a, st);
+        if (N == 128) return ch == 16 ? launch<kMScanHead, 128, 4, 1, 1, 16>(a, st) : launch<kMScanHead, 128, 4, 2, 1, 16>(a, st);
     } else if (mode == kMScanSsd) {
         if (N == 16) return launch<kMScanSsd, 16, 1, 1, 1, 32>(a, st);
         if (N == 32) return launch<kMScanSsd, 32, 2, 1, 1, 32>(a, st);

@@ -2,9 +2,6 @@
 // matrix cores (mfma_scan.hip).
 #pragma once
 
-#include <initializer_list>
-#include <utility>
-
 #include "mi_common.hpp"
 
 namespace mi {
@@ -30,14 +27,9 @@ struct MfmaScanArgs {
     int cs, nchunks_out;     // head mode
 };
 
-// The steps of the first row of a table (rounds up to, steps) that r lies in, 0 past
-// the last: how long sequences a VALU kernel takes instead of the MFMA scan.
-constexpr double kAnyRounds = 1e30;
-inline int steps_at(std::initializer_list<std::pair<double, int>> table, double r) {
-    for (const auto &e : table)
-        if (r <= e.first) return e.second;
-    return 0;
-}
+// The longest sequences that the mode's VALU kernel (scan_kernel, model_scan_kernel,
+// ssd_scan_kernel) takes instead of the MFMA scan; D channels of a row, P of a head.
+int valu_scan_steps(int mode, int N, int B, int D, int P);
 
 // A chunk's rows are addressed by 32-bit byte offsets, so rows stay below this:
 // 64 of them, as int32 outputs, below 2^31 bytes.

@@ -693,18 +693,9 @@ hipError_t launch_ssd_scan(const int8_t *xs, const int8_t *xp, const int8_t *z, 
         }
         return hipGetLastError();
     }
-    // a block of the MFMA scan starts slower (tables, five waves' first loads and
-    // barriers): ssd_scan_kernel up to these steps, by rounds of 16-channel blocks
-    // over CUs (MFMA / this, heads of 64: N16 3 rounds, 8 steps 1.10, 32 steps 0.74, 12
-    // rounds, 48 steps 1.21; N32 3 rounds, 16 steps 1.20, 32 steps 0.89; N64 one round,
-    // 16 steps 1.01, 32 steps 0.81, two rounds, 48 steps 1.04, 64 steps 0.89, 12
-    // rounds, 100 steps 1.03), and for rows too long for the MFMA scan's offsets
-    const double r = (double)B * (a.D / 16) / device_cus();
-    const int steps = N == 16   ? steps_at({{1.9, 4}, {3.9, 12}, {8, 24}, {kAnyRounds, 56}}, r)
-                      : N == 32 ? steps_at({{1, 2}, {2, 8}, {3.9, 16}, {5, 24}, {kAnyRounds, 48}}, r)
-                                : steps_at({{1, 16}, {3.9, 48}, {5, 64}, {9, 80}, {kAnyRounds, 100}}, r);
+    // (short sequences, and rows too long for the MFMA scan's offsets)
     const bool wide = z_row >= kMfmaMaxRow || xp_row >= kMfmaMaxRow;   // (x_row <= z_row)
-    if (wide || L <= steps) {
+    if (wide || L <= valu_scan_steps(kMScanSsd, N, B, a.D, P)) {
         int G = N / 4;
         while (P % (kMThreads / G) != 0) G *= 2;  // P % 16 == 0, so G = 16 always fits
         const dim3 grid((unsigned)(a.D / (kMThreads / G)), (unsigned)B);
@@ -733,21 +724,9 @@ hipError_t launch_model_scan(const int8_t *xs, const int8_t *dm, const int8_t *z
                              const int8_t *csrc, const int32_t *base, int8_t *yo, const int32_t *h_in, int32_t *h_out,
                              int64_t x_row, int64_t z_row, int64_t bc_row, int B, int L, int D, int N, int s_y,
                              hipStream_t st) {
-    // model_scan_kernel where a block of the MFMA scan starts slower than its steps
-    // win back, by rounds of 16-channel blocks over CUs (MFMA / this: N16 1 round, 4
-    // steps 1.02, 8 steps 0.99, 3 rounds, 16 steps 1.05, 8 and 16 rounds, 64 steps 1.07
-    // and 1.09, 100 steps 0.99; N32 1.5 rounds, 100 steps 1.03, 3 rounds, 16 steps 1.02,
-    // 32 steps 0.87, 6 rounds, 64 steps 1.06, 16 rounds, 100 steps 1.11; N64 1 round, 16
-    // steps 1.04, 32 steps 0.94, 2 rounds, 100 steps 1.06), at any length where its
-    // 48-channel blocks make two rounds of 16 channels' four (N32: 1.13 at 400 steps)
-    // and for N = 64 (no model of this size) beyond two rounds (16 rounds, 400 steps
-    // 1.08); and for rows too long for the MFMA scan's offsets
-    const double r = (double)B * ((D + 15) / 16) / device_cus();
-    const int steps = N == 16   ? steps_at({{1, 4}, {2, 12}, {3, 16}, {4.2, 8}, {7, 16}, {9, 64}, {11, 16}, {40, 64}, {kAnyRounds, 112}}, r)
-                      : N == 32 ? steps_at({{1, 4}, {2, 112}, {3, 16}, {4, INT32_MAX}, {7, 64}, {kAnyRounds, 112}}, r)
-                                : steps_at({{1, 24}, {2, 112}, {kAnyRounds, INT32_MAX}}, r);
+    // (model_scan_kernel: short sequences, and rows too long for the MFMA scan's offsets)
     const bool wide = z_row >= kMfmaMaxRow || bc_row >= kMfmaMaxRow;   // (x_row <= z_row)
-    if (!wide && L > steps) {
+    if (!wide && L > valu_scan_steps(kMScanModel, N, B, D, D)) {
         MfmaScanArgs m{};
         m.x = xs; m.dm = dm; m.z = z; m.b = bsrc; m.c = csrc; m.decay = base; m.yo = yo; m.h_in = h_in; m.h_out = h_out;
         m.x_row = x_row; m.z_row = z_row; m.bc_row = bc_row; m.B = B; m.L = L; m.D = D; m.P = D; m.s_y = s_y;
@@ -760,7 +739,7 @@ hipError_t launch_model_scan(const int8_t *xs, const int8_t *dm, const int8_t *z
     auto grid = [&](int ch) { return dim3((unsigned)((D + ch - 1) / ch), (unsigned)B); };
     // (two states a lane while its blocks of 32 channels fill the CUs no more than
     // twice: 2 rounds, 8 steps 4.6 us, 5.3 with four)
-    if (N == 16 && r <= 4.2)
+    if (N == 16 && (double)B * ((D + 15) / 16) <= 4.2 * device_cus())
         hipLaunchKernelGGL((model_scan_kernel<16, 8>), grid(kMThreads / 8), dim3(kMThreads), 0, st, a);
     else if (N == 16)
         hipLaunchKernelGGL((model_scan_kernel<16, 4>), grid(kMThreads / 4), dim3(kMThreads), 0, st, a);

@@ -415,44 +415,20 @@ hipError_t launch_generic(const ScanArgs &a, int N, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Longest sequences that scan_kernel takes, by rounds: 16-channel blocks over CUs.
-// Measured with both kernels over 1 to 128 steps (MFMA / VALU, us a call):
-//   channels  N16   1 round, 1 step 3.6 / 3.0, 8 steps 3.7 / 3.4, 16 steps 4.0 / 3.9,
-//                   32 steps 4.7 / 5.1; 64 rounds, 16 steps 54 / 39, 48 steps 76 / 66
-//             N32   1 round, 8 steps 4.0 / 3.6, 16 steps 4.4 / 4.3
-//             N64   1 round, 8 steps 4.7 / 4.3, 16 steps 5.3 / 5.2; 2 rounds never
-//             N128  3 rounds only (32-channel blocks make one and a half): 8 steps, 1.03 times
-//   heads     N16   6 rounds of 64-channel heads, 16 steps 1.18 times; 3 rounds 0.96
-//             N32   3 rounds 16 steps 1.18; 9 rounds 0.92
-//             N64   1 round 16 steps 1.10; 4.5 rounds 8 steps 1.12, 16 steps 0.92
-//             N128  1 round 8 steps 1.13, 16 steps 0.98; 12 rounds 32 steps 1.03
-int valu_steps(int mode, int N, double r) {
-    if (mode == kModeChannel) {
-        if (N == 16) return steps_at({{1.5, 16}, {4, 8}, {16, 12}, {30, 8}, {45, 24}, {kAnyRounds, 100}}, r);
-        if (N == 32) return steps_at({{1.5, 12}, {3, 4}, {4, 8}, {7, 2}, {8.5, 4}, {11, 2}, {15.5, 4}}, r);
-        if (N == 64) return steps_at({{1, 12}, {1.5, 8}}, r);
-        return steps_at({{2, 0}, {3.9, 8}}, r);
-    }
-    if (N == 16) return steps_at({{2, 16}, {3.9, 12}, {kAnyRounds, 16}}, r);
-    if (N == 32) return steps_at({{1, 16}, {2, 12}, {3.9, 16}, {4.2, 10}, {kAnyRounds, 16}}, r);
-    if (N == 64) return steps_at({{3, 16}, {20, 10}, {kAnyRounds, 16}}, r);
-    return steps_at({{2, 12}, {3, 16}, {7, 8}, {10, 16}, {kAnyRounds, 32}}, r);
-}
-
 // mode channel or head; fast: what mfma_scan_kernel and scan_kernel take but for
 // the row length
 template <int MODE>
 hipError_t launch_scan(const ScanArgs &a, int N, bool fast, hipStream_t st) {
     if (!fast) return launch_generic<MODE>(a, N, st);
     const int64_t row = std::max(a.x_row, a.bc_row);
-    const double r = (double)a.B * a.H * (a.P / 16) / device_cus();
+    const int mode = MODE == kModeChannel ? kMScanChannel : kMScanHead;
     const bool wide = row >= kMfmaMaxRow;
-    if (a.H <= 65535 && (wide || a.L <= valu_steps(MODE, N, r))) return launch_valu_scan<MODE>(a, N, st);   // (heads along y)
+    if (a.H <= 65535 && (wide || a.L <= valu_scan_steps(mode, N, a.B, a.H * a.P, a.P))) return launch_valu_scan<MODE>(a, N, st);   // (heads along y)
     if (wide) return launch_generic<MODE>(a, N, st);
     MfmaScanArgs m{};
     m.x = a.x; m.b = a.bsrc; m.c = a.csrc; m.decay = a.decay; m.y = a.y; m.chunk_states = a.chunk_states; m.h_in = a.h_in; m.h_out = a.h_out;
     m.x_row = a.x_row; m.bc_row = a.bc_row; m.B = a.B; m.L = a.L; m.D = a.H * a.P; m.P = a.P; m.cs = a.cs; m.nchunks_out = a.nchunks_out;
-    return launch_mfma_scan(MODE == kModeChannel ? kMScanChannel : kMScanHead, N, m, st);
+    return launch_mfma_scan(mode, N, m, st);
 }
 
 bool fast_shape(int N, int P, int k, int mode) {

@@ -1,5 +1,5 @@
 """The scans on both sides of their split into the VALU and
-MFMA kernels, by steps and by rounds of 16-channel blocks on 256 CUs, and over rows too
+MFMA kernels, by steps and by rounds of blocks on 256 CUs, and over rows too
 long for the MFMA kernel's offsets, against the CPU oracle (bit for bit)."""
 import numpy as np
 import pytest
@@ -30,7 +30,8 @@ def i32(rng, *shape):
                                            (32, 2, 80, (12, 13, 18, 23, 35)), (32, 5, 2064, (4, 5)), (32, 7, 2064, (8, 9)),
                                            (32, 6, 4096, (2, 3)), (32, 8, 4096, (4, 5)),
                                            (64, 2, 80, (12, 13, 18, 23, 35)), (64, 3, 2048, (8, 9)), (64, 5, 2064, (1, 2)),
-                                           (128, 2, 80, (1, 9, 15, 18, 35)), (128, 6, 2064, (8, 9))])
+                                           (128, 2, 80, (1, 9, 15, 18, 35)), (128, 6, 2064, (8, 9)),
+                                           (16, 1, 4096, (16, 17)), (32, 7, 2064, (22, 23)), (64, 4, 2048, (6, 7)), (128, 6, 2064, (14, 15))])
 def test_channel_routes(cuda, n, b, d, lengths):
     from mamba_int import ops
     rng = np.random.default_rng(n + b + d)
@@ -48,7 +49,9 @@ def test_channel_routes(cuda, n, b, d, lengths):
                                                  (32, 2, 3, 48, (16, 17, 22, 35)), (32, 8, 24, 64, (16, 17)), (32, 12, 24, 64, (16,)),
                                                  (32, 24, 24, 64, (16,)), (32, 44, 24, 64, (16, 17)),
                                                  (64, 2, 5, 16, (16, 17, 22, 35)), (64, 12, 24, 64, (10, 11)), (64, 24, 24, 64, (10, 11)),
-                                                 (128, 2, 3, 48, (12, 13)), (128, 8, 24, 64, (16, 17)), (128, 32, 24, 64, (32, 33))])
+                                                 (128, 2, 3, 48, (12, 13)), (128, 8, 24, 64, (16, 17)), (128, 32, 24, 64, (32, 33)),
+                                                 (16, 12, 24, 64, (17,)), (64, 2, 5, 16, (28, 29)), (128, 6, 16, 48, (64, 65)),
+                                                 (128, 8, 24, 64, (28, 29))])
 def test_head_routes(cuda, n, b, heads, p, lengths):
     import torch
     from mamba_int import ops
@@ -58,7 +61,7 @@ def test_head_routes(cuda, n, b, heads, p, lengths):
         x, bb, cc = i8(rng, b, length, heads, p), i8(rng, b, length, heads, n), i8(rng, b, length, heads, n)
         h = i32(rng, b, heads, p, n)
         y_ref, st_ref, h_ref = O.ssd_chunked_scan(x, bb, cc, nd, 15, 64, h_state=h.copy(), want_chunk_states=True)
-        ht, st = T(h), torch.empty((b, 1, heads, p, n), dtype=torch.int32, device="cuda")
+        ht, st = T(h), torch.empty((b, -(-length // 64), heads, p, n), dtype=torch.int32, device="cuda")
         y = ops.ssd_chunked_scan(T(x), T(bb), T(cc), T(nd), 15, 64, chunk_states=st, h_in=ht, h_out=ht)
         for got, want in ((y, y_ref), (st, st_ref), (ht, h_ref)):
             assert np.array_equal(got.cpu().numpy(), want), length
@@ -95,7 +98,8 @@ def test_block_scan_long_rows(cuda, n, length):
 @pytest.mark.parametrize("n,b,d,lengths", [(16, 2, 80, (4, 5)), (16, 4, 2048, (12, 13)), (16, 6, 2064, (16, 17)), (16, 8, 2048, (8, 9)),
                                            (16, 9, 2064, (16, 17)), (16, 16, 2064, (64, 65)), (32, 2, 80, (4, 5)),
                                            (32, 4, 2048, (112, 113)), (32, 6, 2064, (16, 200)), (32, 9, 2064, (64, 65)),
-                                           (64, 2, 80, (24, 25)), (64, 4, 2048, (112, 113)), (64, 5, 2064, (150,))])
+                                           (64, 2, 80, (24, 25, 28, 29)), (64, 4, 2048, (112, 113, 160, 161)), (64, 5, 2064, (150,)),
+                                           (16, 3, 4112, (24, 25)), (16, 14, 2064, (64, 65)), (32, 5, 2048, (24, 25)), (32, 9, 2048, (80, 81))])
 def test_block_routes(cuda, n, b, d, lengths):
     from mamba_int import ops
     rng = np.random.default_rng(n + b + d)
@@ -112,7 +116,9 @@ def test_block_routes(cuda, n, b, d, lengths):
 @pytest.mark.parametrize("n,b,heads,p,lengths", [(16, 2, 3, 48, (4, 5)), (16, 4, 8, 64, (12, 13)), (16, 20, 24, 64, (56, 57)),
                                                  (32, 2, 3, 48, (2, 3)), (32, 8, 24, 64, (16, 17)), (32, 20, 24, 64, (48, 49)),
                                                  (64, 2, 3, 48, (16, 17)), (64, 4, 24, 64, (48, 49)), (64, 12, 24, 64, (64, 65)),
-                                                 (64, 16, 24, 64, (80, 81)), (64, 26, 24, 64, (100, 101))])
+                                                 (64, 16, 24, 64, (80, 81)), (64, 26, 24, 64, (100, 101)),
+                                                 (16, 8, 24, 64, (12, 13)), (32, 8, 24, 64, (28, 29)), (64, 4, 24, 64, (64, 65)),
+                                                 (64, 20, 24, 64, (128, 129))])
 def test_ssd_routes(cuda, n, b, heads, p, lengths):
     from mamba_int import ops
     rng = np.random.default_rng(n + b + heads)
