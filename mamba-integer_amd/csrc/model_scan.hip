@@ -2,9 +2,9 @@
 // decay from base + dm, dt from dm, input xs*dt (x) B, the exact floor
 // recurrence, y = C.h, the gate by z and the requant of the out_proj input.
 //
-// (mfma_scan.hip has the form that most shapes take; this one remains for short
-// sequences, where launch_model_scan measured it faster, and for N = 64 at many
-// channels.)
+// (mfma_scan.hip has the form that most shapes take; this one remains where
+// valu_scan_steps there measured it faster: short sequences, and some block counts at
+// any length, N = 64 beyond two rounds among them.)
 //
 // Layout: a block of 256 threads owns CH = 256/G channels of one sequence; G
 // adjacent lanes share a channel and keep S = N/G states each in VGPRs (read
